@@ -9,7 +9,7 @@
 //                     (include/green_dyadic.hxx:112-288, SHOprj), sum-factorised, split into
 //                     chunks of blocks whose partial sums are reduced in a fixed order;
 //   2. k_sho_atoms    collect images -> atom with Bloch phases, multiply the atom matrix
-//                     (h - E s) dVol, broadcast back with conjugate phases
+//                     (h - E s) dVol on the matrix cores, broadcast back with conjugate phases
 //                     (include/green_dyadic.hxx:600-852, SHOsum + SHOmul + SHOsum);
 //   3. the local kernel, per (block, column slice): (V - E) x (include/green_potential.hxx:16-139) + the
 //                     three finite-difference Laplacians (include/green_kinetic.hxx:24-329) + the SHO add-back
@@ -299,76 +299,152 @@ __global__ __launch_bounds__(256) void k_sho_project_mfma(
 }
 
 // ---------------------------------------------------------------------------------------------
-// 2. per (atom, column): collect images with phase, multiply (h - E s) dVol, broadcast with
-//    conjugate phase.  ATOM_WAVES waves; lane = column j, both planes per thread.  The waves share
-//    the collected coefficients (LDS up to 64 coefficients, numax <= 5, else a global scratch row):
-//    coefficient s is collected by wave s % ATOM_WAVES, output row i computed by wave i % ATOM_WAVES.
+// 2. per (atom, column): collect images with phase, multiply (h - E s) dVol, broadcast with conjugate phase.
+//    The 64 right-hand sides of a column group are independent, so a work-group takes JS of them for one (atom,
+//    column): 512 threads collect the chunk partial sums into LDS (thread = one right-hand side of one coefficient,
+//    both planes), then the waves multiply on the matrix cores.  h and s are real, so with the collected c = (c_re,
+//    c_im) the products t = h c and u = s c are real contractions, [16 rows of h and s] x [nc] x [16 right-hand sides
+//    of both planes] per wave on the FP64 16x16x4 MFMA (operand layout as in k_sho_project_mfma), and d = t - E u.
+//    Bound by latency: a plan has few (atom, column) pairs, and one pair's chain (chunk list, partial sums, matrix)
+//    is what a launch takes.  The chunks of a pair are therefore one list in memory, read ahead of the sums, the
+//    first 64 columns of the wave's matrix rows are loaded before the collection, and JS is small enough for four
+//    (two) work-groups per pair.  Measured, against one work-group of 8 waves per pair on the vector ALUs that read
+//    chunk by chunk: FP64 numax 5, 215 pairs: 212 -> 73 us; numax 7, 16 pairs: 428 -> 46 us; numax 2, 2 pairs of 13
+//    images: 63 -> 19 us; FP32 numax 5, 1,370 pairs: 309 -> 164 us.  Holding the kernel to 128 VGPRs (4 waves per
+//    SIMD instead of 3) spills and takes 96, 55, 22 and 225 us.
 // ---------------------------------------------------------------------------------------------
-#define ATOM_WAVES 8
+// one chunk of the projection partial sums of an (atom, column): its first coefficient row and its atom image
+struct CollectEntry {
+    uint32_t coef, img;
+};
+
+// adds U chunks from e0 on (those below e1) to the sum below; their loads are in flight together
+template <typename real_t, int U>
+__device__ __forceinline__ void collect_chunks(real_t const* __restrict__ partial,
+                                               CollectEntry const* __restrict__ coll, uint32_t e0, uint32_t e1,
+                                               double const* __restrict__ image_phase, int s, int j, double& ar,
+                                               double& ai) {
+    double vr[U], vi[U], pr[U], pi[U];
+#pragma unroll
+    for (int q = 0; q < U; ++q) {   // beyond the end: the last chunk again, not added
+        CollectEntry const en = coll[min(e0 + q, e1 - 1)];
+        real_t const* src = partial + (size_t(en.coef) + s) * 128 + j;
+        vr[q] = double(src[0]);
+        vi[q] = double(src[64]);
+        pr[q] = image_phase[2 * en.img];
+        pi[q] = image_phase[2 * en.img + 1];
+    }
+#pragma unroll
+    for (int q = 0; q < U; ++q)
+        if (e0 + q < e1) {
+            ar += pr[q] * vr[q] - pi[q] * vi[q];
+            ai += pr[q] * vi[q] + pi[q] * vr[q];
+        }
+}
+
+// sum over the chunks e0 .. e1 - 1 of an (atom, column) of the partial sums of coefficient s at right-hand side j,
+// each with the Bloch phase of its image, in list order
 template <typename real_t>
-__global__ __launch_bounds__(64 * ATOM_WAVES) void k_sho_atoms(
-    real_t* __restrict__ dcoef, real_t const* __restrict__ partial, uint32_t const* __restrict__ chunk_coef,
-    uint32_t const* __restrict__ pair_chunk, uint32_t const* __restrict__ sum_start,
-    uint32_t const* __restrict__ sum_index, uint32_t const* __restrict__ image_starts,
+__device__ __forceinline__ void collect_coefficient(real_t const* __restrict__ partial,
+                                                    CollectEntry const* __restrict__ coll, uint32_t e0, uint32_t e1,
+                                                    double const* __restrict__ image_phase, int s, int j, double& ar,
+                                                    double& ai) {
+    ar = ai = 0;
+    uint32_t e = e0;
+    for (; e + 8 < e1; e += 16) collect_chunks<real_t, 16>(partial, coll, e, e1, image_phase, s, j, ar, ai);
+    if (e < e1) collect_chunks<real_t, 8>(partial, coll, e, e1, image_phase, s, j, ar, ai);
+}
+
+constexpr int ATOM_T = 512;   // threads of k_sho_atoms
+
+template <typename real_t, int JS>
+__global__ __launch_bounds__(ATOM_T) void k_sho_atoms(
+    real_t* __restrict__ dcoef, real_t const* __restrict__ partial, uint32_t const* __restrict__ pairs,
+    uint32_t const* __restrict__ coll_start, CollectEntry const* __restrict__ coll,
+    uint32_t const* __restrict__ sum_start, uint32_t const* __restrict__ sum_index,
+    uint32_t const* __restrict__ image_starts,
     int8_t const* __restrict__ atom_lmax, double const* __restrict__ atom_mat,
     uint64_t const* __restrict__ atom_mat_off, double const* __restrict__ image_phase, uint32_t nCols,
-    double* __restrict__ cscratch, uint32_t const* __restrict__ atom_starts, double const* __restrict__ E_col,
-    uint8_t const* __restrict__ col_active) {
-    extern __shared__ double lds[];
-    uint32_t const a = blockIdx.x, c = blockIdx.y;
+    double const* __restrict__ E_col, uint8_t const* __restrict__ col_active) {
+    using acc_t = typename Mfma<double>::acc_t;
+    constexpr int NS = 64 / JS, NJ = JS / 16;   // slices per pair, 16-column tiles per plane
+    constexpr int KA = 16;                      // k-steps (of 4 columns of h and s) loaded together
+    extern __shared__ double cs[];              // [plane][16-column tile][coefficient, padded to 4][16]
+    // the pairs with a block of the column near the atom: those of small truncation spheres see few of the atoms,
+    // and the coefficients of the others are never read
+    uint32_t const slice = blockIdx.x % NS, pair = pairs[blockIdx.x / NS], c = pair % nCols, a = pair / nCols;
     if (col_active && !col_active[c]) return;  // a retired column group
-    // the wave index is uniform: the rows i = w, w + ATOM_WAVES, ... of M are read with scalar loads
-    int const j = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    uint32_t const e0 = coll_start[pair], e1 = coll_start[pair + 1];
+    int const tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int const n = lane & 15, kl = lane >> 4;
     int const L = atom_lmax[a];
-    int const nc = ((L + 1) * (L + 2) * (L + 3)) / 6;
-    bool const in_lds = nc <= 64;
-    double* cre = in_lds ? lds : cscratch + (size_t(atom_starts[a]) * nCols + size_t(c) * nc) * 128;
-    double* cim = cre + nc * 64;
+    int const nc = ((L + 1) * (L + 2) * (L + 3)) / 6, kp = (nc + 3) & ~3, nks = kp / 4, nu = ((nc + 15) / 16) * NJ;
     double const* HS = atom_mat + atom_mat_off[a];  // [2][nc][nc]: h dVol, s dVol
     double const Er = E_col[2 * c], Ei = E_col[2 * c + 1];
-    uint32_t const k0 = sum_start[a], k1 = sum_start[a + 1];
-    for (int s = w; s < nc; s += ATOM_WAVES) {
-        double ar = 0, ai = 0;
-        for (uint32_t k = k0; k < k1; ++k) {
-            uint32_t const img = sum_index[k];
-            double const ph_re = image_phase[2 * img], ph_im = image_phase[2 * img + 1];
-            uint32_t const c0 = pair_chunk[size_t(img) * nCols + c], c1 = pair_chunk[size_t(img) * nCols + c + 1];
-            double vr = 0, vi = 0;
-            for (uint32_t ch = c0; ch < c1; ++ch) {
-                real_t const* src = partial + (size_t(chunk_coef[ch]) + s) * 128 + j;
-                vr += double(src[0]);
-                vi += double(src[64]);
-            }
-            ar += ph_re * vr - ph_im * vi;
-            ai += ph_re * vi + ph_im * vr;
-        }
-        if (in_lds) { lds[s * 64 + j] = ar; lds[(nc + s) * 64 + j] = ai; }   // LDS addressed as such
-        else { cre[s * 64 + j] = ar; cim[s * 64 + j] = ai; }
-    }
-    __syncthreads();
-    // d = M c with M = (h - E s) dVol of this column's energy, complex double accumulation in ascending
-    // column order (include/green_dyadic.hxx:800-819, src/green_function.cxx:97-98); the rows of M are
-    // wave-uniform (scalar loads), the coefficients per column come from LDS (numax <= 5) or the scratch
-    auto mv = [&](int i, double const* __restrict__ cr_, double const* __restrict__ ci_, double& dr, double& di) {
-#pragma unroll 4
-        for (int k = 0; k < nc; ++k) {
-            double const hd = HS[i * nc + k], sd = HS[nc * nc + i * nc + k];
-            double const mr = hd - Er * sd, mi = -Ei * sd;
-            double const cr = cr_[k * 64 + j], ci = ci_[k * 64 + j];
-            dr += mr * cr - mi * ci;
-            di += mr * ci + mi * cr;
+
+    double ah[KA], as[KA];   // the wave's rows of h and s: A[m = n][k = ks * 4 + kl]
+    auto load_rows = [&](int mt, int ks0) {
+        int const i = mt * 16 + n;
+#pragma unroll
+        for (int q = 0; q < KA; ++q) {
+            int const k = (ks0 + q) * 4 + kl;
+            bool const in = i < nc && k < nc;
+            int const at = in ? i * nc + k : 0;
+            double const h = HS[at], sv = HS[nc * nc + at];
+            ah[q] = in ? h : 0.0;
+            as[q] = in ? sv : 0.0;
         }
     };
-    for (int i = w; i < nc; i += ATOM_WAVES) {
-        double dr = 0, di = 0;
-        if (in_lds) mv(i, lds, lds + nc * 64, dr, di);
-        else mv(i, cre, cim, dr, di);
+    if (w < nu) load_rows(w / NJ, 0);
+
+    for (int s = tid / JS; s < kp; s += ATOM_T / JS) {
+        int const jl = tid % JS;
+        double ar = 0, ai = 0;
+        if (s < nc) collect_coefficient<real_t>(partial, coll, e0, e1, image_phase, s, slice * JS + jl, ar, ai);
+        cs[((jl >> 4) * kp + s) * 16 + (jl & 15)] = ar;
+        cs[((NJ + (jl >> 4)) * kp + s) * 16 + (jl & 15)] = ai;
+    }
+    __syncthreads();
+
+    uint32_t const k0 = sum_start[a], k1 = sum_start[a + 1];
+    for (int u = w; u < nu; u += ATOM_T / 64) {
+        int const mt = u / NJ, jt = u % NJ;
+        acc_t tr = {0, 0, 0, 0}, ti = {0, 0, 0, 0}, ur = {0, 0, 0, 0}, ui = {0, 0, 0, 0};
+        double const* cr = cs + jt * kp * 16 + n;
+        double const* ci = cs + (NJ + jt) * kp * 16 + n;
+        for (int ks0 = 0; ks0 < nks; ks0 += KA) {
+            if (u != w || ks0 > 0) load_rows(mt, ks0);
+#pragma unroll
+            for (int q = 0; q < KA; ++q) {
+                if (ks0 + q < nks) {   // uniform
+                    int const k = (ks0 + q) * 4 + kl;
+                    double const br = cr[k * 16], bi = ci[k * 16];
+                    tr = Mfma<double>::mac(ah[q], br, tr);
+                    ti = Mfma<double>::mac(ah[q], bi, ti);
+                    ur = Mfma<double>::mac(as[q], br, ur);
+                    ui = Mfma<double>::mac(as[q], bi, ui);
+                }
+            }
+        }
+        // d = t - E u (include/green_dyadic.hxx:800-819, src/green_function.cxx:97-98), then every image's share
+        double dr[4], di[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            dr[r] = tr[r] - (Er * ur[r] - Ei * ui[r]);
+            di[r] = ti[r] - (Er * ui[r] + Ei * ur[r]);
+        }
         for (uint32_t k = k0; k < k1; ++k) {
             uint32_t const img = sum_index[k];
             double const ph_re = image_phase[2 * img], ph_im = -image_phase[2 * img + 1];
-            real_t* dst = dcoef + ((size_t(image_starts[img]) + i) * nCols + c) * 128 + j;
-            dst[0] = real_t(ph_re * dr - ph_im * di);
-            dst[64] = real_t(ph_re * di + ph_im * dr);
+            real_t* dst = dcoef + (size_t(image_starts[img]) * nCols + c) * 128 + slice * JS + jt * 16 + n;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                int const i = mt * 16 + Mfma<double>::row(kl, r);
+                if (i < nc) {
+                    dst[size_t(i) * nCols * 128] = real_t(ph_re * dr[r] - ph_im * di[r]);
+                    dst[size_t(i) * nCols * 128 + 64] = real_t(ph_re * di[r] + ph_im * dr[r]);
+                }
+            }
         }
     }
 }
@@ -1733,7 +1809,35 @@ int device_upload_plan(Plan const& p, DevicePlan& d, std::string& err) {
             d.slot_map.clear();
         }
         if ((s = dupload(d, d.chunk_coef, coef, err))) return s;
-        if ((s = dupload(d, d.pair_chunk, pair_chunk, err))) return s;
+        {   // the chunks of every (atom, column) in one list, images in the order of the collection; one upload of
+            // [start of every pair | chunks | pairs with chunks]
+            size_t const npair = size_t(p.nAtoms) * p.nCols;
+            std::vector<uint32_t> t, list, pairs;
+            t.reserve(2 * npair + 1 + 2 * chunks.size());
+            list.reserve(2 * chunks.size());
+            t.push_back(0);
+            for (uint32_t a = 0; a < p.nAtoms; ++a)
+                for (uint32_t c = 0; c < p.nCols; ++c) {
+                    for (uint32_t k = p.sho_sum.start[a]; k < p.sho_sum.start[a + 1]; ++k) {
+                        uint32_t const img = p.sho_sum.index[k];
+                        size_t const ic = size_t(img) * p.nCols + c;
+                        for (uint32_t ch = pair_chunk[ic]; ch < pair_chunk[ic + 1]; ++ch) {
+                            list.push_back(coef[ch]);
+                            list.push_back(img);
+                        }
+                    }
+                    if (list.size() / 2 > t.back()) pairs.push_back(uint32_t(t.size() - 1));
+                    t.push_back(uint32_t(list.size() / 2));
+                }
+            if (t.size() & 1) t.push_back(0);   // the 8-byte chunk records start on 8 bytes
+            size_t const at_list = t.size(), at_pairs = at_list + list.size();
+            t.insert(t.end(), list.begin(), list.end());
+            t.insert(t.end(), pairs.begin(), pairs.end());
+            if ((s = dupload(d, d.coll_start, t, err))) return s;
+            d.coll = d.coll_start + at_list;
+            d.atom_pairs = d.coll_start + at_pairs;
+            d.n_atom_pairs = uint32_t(pairs.size());
+        }
         if ((s = dupload(d, d.bucket_chunks, bucket, err))) return s;
     }
 
@@ -1794,35 +1898,21 @@ __global__ __launch_bounds__(64) void k_grad_v_cells(double* __restrict__ gcell,
 }
 
 // atom coefficients of one vector: per (atom, column group) the image partials collected with the Bloch phase,
-// out[((atom_starts[a] + s) * nCols + c)][re/im][j] (the input of the atom-matrix multiply of k_sho_atoms)
-__global__ __launch_bounds__(64 * ATOM_WAVES) void k_sho_collect(
-    double* __restrict__ out, double const* __restrict__ partial, uint32_t const* __restrict__ chunk_coef,
-    uint32_t const* __restrict__ pair_chunk, uint32_t const* __restrict__ sum_start,
-    uint32_t const* __restrict__ sum_index, int8_t const* __restrict__ atom_lmax,
+// out[((atom_starts[a] + s) * nCols + c)][re/im][j] (the input of the atom-matrix multiply of k_sho_atoms).  One
+// work-group per (atom, column, 4 coefficients), a wave per coefficient.
+__global__ __launch_bounds__(256) void k_sho_collect(
+    double* __restrict__ out, double const* __restrict__ partial, uint32_t const* __restrict__ coll_start,
+    CollectEntry const* __restrict__ coll, int8_t const* __restrict__ atom_lmax,
     double const* __restrict__ image_phase, uint32_t nCols, uint32_t const* __restrict__ atom_starts) {
-    uint32_t const a = blockIdx.x, c = blockIdx.y;
-    int const j = threadIdx.x & 63, w = threadIdx.x >> 6;
+    uint32_t const pair = blockIdx.x, c = pair % nCols, a = pair / nCols;
+    int const j = threadIdx.x & 63, s = blockIdx.y * 4 + (threadIdx.x >> 6);
     int const L = atom_lmax[a];
-    int const nc = ((L + 1) * (L + 2) * (L + 3)) / 6;
-    for (int s = w; s < nc; s += ATOM_WAVES) {
-        double ar = 0, ai = 0;
-        for (uint32_t k = sum_start[a]; k < sum_start[a + 1]; ++k) {
-            uint32_t const img = sum_index[k];
-            double const ph_re = image_phase[2 * img], ph_im = image_phase[2 * img + 1];
-            uint32_t const c0 = pair_chunk[size_t(img) * nCols + c], c1 = pair_chunk[size_t(img) * nCols + c + 1];
-            double vr = 0, vi = 0;
-            for (uint32_t ch = c0; ch < c1; ++ch) {
-                double const* src = partial + (size_t(chunk_coef[ch]) + s) * 128 + j;
-                vr += src[0];
-                vi += src[64];
-            }
-            ar += ph_re * vr - ph_im * vi;
-            ai += ph_re * vi + ph_im * vr;
-        }
-        double* dst = out + ((size_t(atom_starts[a]) + s) * nCols + c) * 128 + j;
-        dst[0] = ar;
-        dst[64] = ai;
-    }
+    if (s >= ((L + 1) * (L + 2) * (L + 3)) / 6) return;
+    double ar, ai;
+    collect_coefficient<double>(partial, coll, coll_start[pair], coll_start[pair + 1], image_phase, s, j, ar, ai);
+    double* dst = out + ((size_t(atom_starts[a]) + s) * nCols + c) * 128 + j;
+    dst[0] = ar;
+    dst[64] = ai;
 }
 
 // per (atom a, row k): for every l, z_c = sum_j conj(cL[k][c][j]) cX[l][c][j];
@@ -1900,7 +1990,7 @@ template <> Workspace<float>& workspace<float>(DevicePlan& d) { return d.ws32; }
 
 template <typename real_t>
 int device_action(DevicePlan& d, ActionScalars const& s, real_t* y, real_t const* x, hipStream_t stream,
-                  std::string& err, int parts, double* dot, Workspace<real_t>* ext, double* ext_cscratch) {
+                  std::string& err, int parts, double* dot, Workspace<real_t>* ext) {
     auto& ws = ext ? *ext : workspace<real_t>(d);
     if (!ext) {
         // every buffer of this precision is allocated on the first call, so that later calls (also under graph
@@ -1909,19 +1999,10 @@ int device_action(DevicePlan& d, ActionScalars const& s, real_t* y, real_t const
             if (int r = dalloc(d, ws.partial, size_t(d.total_chunk_coefs) * 128, err)) return r;
             if (int r = dalloc(d, ws.dcoef, size_t(d.natomcoeffs) * d.nCols * 128, err)) return r;
         }
-        if (d.nAtomImages > 0 && d.nchunks > 0 && d.max_atom_nc > 64 && !d.cscratch) {
-            if (int r = dalloc(d, d.cscratch, size_t(d.ncoeffs) * d.nCols * 128, err)) return r;
-        }
         if (!ws.zero) {
             if (int r = dalloc(d, ws.zero, NBLK, err)) return r;
             HIP_TRY(hipMemsetAsync(ws.zero, 0, NBLK * sizeof(real_t), stream));
         }
-    }
-    // after the allocations above: the atom-multiply scratch of numax 6, 7 atoms exists from here on
-    double* const cscratch = ext ? ext_cscratch : d.cscratch;
-    if ((parts & ACTION_PROJECT) && d.nAtomImages > 0 && d.nchunks > 0 && d.max_atom_nc > 64 && !cscratch) {
-        err = "no scratch for the atom matrices of numax 6, 7 atoms";
-        return 1;
     }
     if ((parts & ACTION_PROJECT) && d.nAtomImages > 0 && d.nchunks > 0) {
         for (int L = 0; L <= 7; ++L) {
@@ -1951,12 +2032,19 @@ int device_action(DevicePlan& d, ActionScalars const& s, real_t* y, real_t const
 #undef LAUNCH_MFMA
             HIP_TRY(hipGetLastError());
         }
-        uint32_t const ncl = std::min<uint32_t>(d.max_atom_nc, 64);   // larger atoms use the global scratch
-        size_t const lds = size_t(2) * ncl * 64 * sizeof(double);
-        hipLaunchKernelGGL((k_sho_atoms<real_t>), dim3(d.nAtoms, d.nCols), dim3(64 * ATOM_WAVES), lds, stream, ws.dcoef,
-                           ws.partial, d.chunk_coef, d.pair_chunk, d.sum_start, d.sum_index, d.image_starts,
-                           d.atom_lmax, d.atom_hs, d.atom_mat_off, d.image_phase, d.nCols, cscratch,
-                           d.atom_starts, d.E_col, d.col_active);
+        // right-hand sides per work-group: 16 fill 128-byte lines in FP64; in FP32 32 do (1,370 pairs: 164 us
+        // against 182 us with 16), and 16 (twice the work-groups, half lines) are taken while 32 would leave CUs
+        // idle, below 512 pairs = 1,024 work-groups
+        uint64_t const pairs = d.n_atom_pairs;
+        int const JS = (sizeof(real_t) == 4 && pairs >= 512) ? 32 : 16;
+        if (pairs * (64 / JS) > 0x7fffffffull) { err = "too many (atom, column) pairs for one launch"; return 1; }
+        size_t const lds = size_t(2) * JS * ((d.max_atom_nc + 3) & ~3u) * sizeof(double);
+#define LAUNCH_ATOMS(JS_) hipLaunchKernelGGL((k_sho_atoms<real_t, JS_>), dim3(uint32_t(pairs) * (64 / JS_)), \
+            dim3(ATOM_T), lds, stream, ws.dcoef, ws.partial, d.atom_pairs, d.coll_start, \
+            reinterpret_cast<CollectEntry const*>(d.coll), d.sum_start, d.sum_index, d.image_starts, d.atom_lmax, d.atom_hs, d.atom_mat_off, d.image_phase, d.nCols, \
+            d.E_col, d.col_active)
+        if (JS == 32) LAUNCH_ATOMS(32); else LAUNCH_ATOMS(16);
+#undef LAUNCH_ATOMS
         HIP_TRY(hipGetLastError());
     }
     if (!(parts & ACTION_LOCAL)) return 0;
@@ -2019,14 +2107,13 @@ int device_action(DevicePlan& d, ActionScalars const& s, real_t* y, real_t const
 }
 
 template int device_action<double>(DevicePlan&, ActionScalars const&, double*, double const*, hipStream_t, std::string&,
-                                   int, double*, Workspace<double>*, double*);
+                                   int, double*, Workspace<double>*);
 template int device_action<float>(DevicePlan&, ActionScalars const&, float*, float const*, hipStream_t, std::string&,
-                                  int, double*, Workspace<float>*, double*);
+                                  int, double*, Workspace<float>*);
 
 // ---------------------------------------------------------------------------------------------
-// The action without allocation (gfa_action_noalloc): the projection partial sums, the addition coefficients,
-// the atom-multiply scratch of numax 6, 7 atoms and the zero block live in `scratch`, a fixed array of every GPU
-// the library runs on (held until the process ends).  Its device address is taken once per device with
+// The action without allocation (gfa_action_noalloc): the projection partial sums, the addition coefficients
+// and the zero block live in `scratch`, a fixed array of every GPU the library runs on (held until the process ends).  Its device address is taken once per device with
 // hipGetSymbolAddress; the host-side name `scratch` is never handed to a kernel.  Calls that overlap on one GPU
 // share the array and race.
 // ---------------------------------------------------------------------------------------------
@@ -2071,6 +2158,8 @@ size_t noalloc_scratch_bytes(DevicePlan const& d, int fp_bits) {
     if (d.nAtomImages > 0) {
         b += round256(size_t(d.total_chunk_coefs) * 128 * s);
         b += round256(size_t(d.natomcoeffs) * d.nCols * 128 * s);
+        // one FP64 row per collected coefficient of a plan with numax 6, 7 atoms: no longer stored, but the plans the
+        // allocation-free action takes stay the same
         if (d.nchunks > 0 && d.max_atom_nc > 64) b += round256(size_t(d.ncoeffs) * d.nCols * 128 * 8);
     }
     return b;
@@ -2091,18 +2180,15 @@ int device_action_noalloc(DevicePlan& d, ActionScalars const& s, real_t* y, real
     auto take = [&](size_t bytes) { unsigned char* p = cur; cur += round256(bytes); return p; };
     Workspace<real_t> ws;
     ws.zero = reinterpret_cast<real_t*>(take(size_t(NBLK) * sizeof(real_t)));
-    double* csc = nullptr;
     if (d.nAtomImages > 0) {
         ws.partial = reinterpret_cast<real_t*>(take(size_t(d.total_chunk_coefs) * 128 * sizeof(real_t)));
         ws.dcoef = reinterpret_cast<real_t*>(take(size_t(d.natomcoeffs) * d.nCols * 128 * sizeof(real_t)));
-        if (d.nchunks > 0 && d.max_atom_nc > 64)
-            csc = reinterpret_cast<double*>(take(size_t(d.ncoeffs) * d.nCols * 128 * 8));
     }
     // the array keeps the previous call's contents: the zero block is cleared on every call (a kernel, so that
     // the call can be captured in a graph); the other regions are written before they are read
     hipLaunchKernelGGL((k_fill_zero<real_t>), dim3((NBLK + 255) / 256), dim3(256), 0, stream, ws.zero, uint32_t(NBLK));
     HIP_TRY(hipGetLastError());
-    return device_action<real_t>(d, s, y, x, stream, err, ACTION_ALL, nullptr, &ws, csc);
+    return device_action<real_t>(d, s, y, x, stream, err, ACTION_ALL, nullptr, &ws);
 }
 template int device_action_noalloc<double>(DevicePlan&, ActionScalars const&, double*, double const*, hipStream_t,
                                            std::string&);
@@ -2207,9 +2293,9 @@ static int project_collect(DevicePlan& d, ActionScalars const& s, double const* 
         }
 #undef LAUNCH_PRJ
     }
-    hipLaunchKernelGGL(k_sho_collect, dim3(d.nAtoms, d.nCols), dim3(64 * ATOM_WAVES), 0, stream, out, ws.partial,
-                       d.chunk_coef, d.pair_chunk, d.sum_start, d.sum_index, d.atom_lmax, d.image_phase, d.nCols,
-                       d.atom_starts);
+    hipLaunchKernelGGL(k_sho_collect, dim3(d.nAtoms * d.nCols, (d.max_atom_nc + 3) / 4), dim3(256), 0, stream, out,
+                       ws.partial, d.coll_start, reinterpret_cast<CollectEntry const*>(d.coll), d.atom_lmax,
+                       d.image_phase, d.nCols, d.atom_starts);
     HIP_TRY(hipGetLastError());
     return 0;
 }

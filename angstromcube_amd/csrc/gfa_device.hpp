@@ -88,14 +88,16 @@ struct DevicePlan {
     ProjChunk* chunks = nullptr;       // [nchunks]
     uint32_t* chunk_coef = nullptr;    // [nchunks+1] coefficient offsets of the partial sums
     uint32_t* prj_blocks = nullptr;    // flat inzb lists of all chunks
-    uint32_t* pair_chunk = nullptr;    // [nai*nCols+1] chunk range of each (image, column)
+    uint32_t* coll_start = nullptr;    // [nAtoms*nCols+1] range of each (atom, column) in coll
+    uint32_t* atom_pairs = nullptr;    // [n_atom_pairs] a * nCols + c of the (atom, column) pairs with chunks
+    uint32_t n_atom_pairs = 0;
+    uint32_t* coll = nullptr;          // [chunks][2] first coefficient row and atom image of its chunks
     uint32_t* bucket_chunks = nullptr; // chunk ids sorted by numax
     uint32_t bucket_start[9] = {0};    // ranges into bucket_chunks per numax 0..7
     uint32_t* sum_start = nullptr;     // [nAtoms+1]
     uint32_t* sum_index = nullptr;
     int8_t* atom_lmax = nullptr;       // [nAtoms]
     uint32_t* atom_starts = nullptr;   // [nAtoms+1]
-    double* cscratch = nullptr;        // [ncoeffs * nCols][2][64] atom coefficients when numax > 5
     uint64_t ncoeffs = 0;
     uint32_t max_atom_nc = 0;
     uint32_t nchunks = 0;
@@ -141,12 +143,10 @@ void device_free(DevicePlan& d);
 // parts of the action: the SHO projection and atom-matrix multiply (coefficients into the workspace), and
 // the local kernel (potential, kinetic, add-back of the workspace coefficients) that writes y
 enum { ACTION_PROJECT = 1, ACTION_LOCAL = 2, ACTION_ALL = 3 };
-// ext: a workspace the caller provides (no buffer of the plan is allocated or used); ext_cscratch its atom-multiply
-// scratch for numax 6, 7 atoms
+// ext: a workspace the caller provides (no buffer of the plan is allocated or used)
 template <typename real_t>
 int device_action(DevicePlan& d, ActionScalars const& s, real_t* y, real_t const* x, hipStream_t stream,
-                  std::string& err, int parts = ACTION_ALL, double* dot = nullptr, Workspace<real_t>* ext = nullptr,
-                  double* ext_cscratch = nullptr);
+                  std::string& err, int parts = ACTION_ALL, double* dot = nullptr, Workspace<real_t>* ext = nullptr);
 
 // the whole action with its workspace in the library's fixed per-device scratch array (no allocation); the plan
 // must be on the device already.  Returns 1 if the plan needs more than NOALLOC_SCRATCH_BYTES.
