@@ -10,7 +10,7 @@
 //
 // Layout of the work: one full TFQMR step (an even and an odd half-step, two actions) is
 //     alpha | K_even | theta_e | A un | K_odd | theta_o | K_dx2 | A u | K_vnext
-// where the K_* kernels stream the vectors of one segment (<= SEG blocks of one column group) per
+// where the K_* kernels stream the vectors of one segment (a few blocks of one column group) per
 // work-group and leave their inner-product partials per segment; the scalar kernels fold the segments of
 // a column in a fixed order, so every reduction is deterministic.  The two x updates of a step are
 // deferred into one pass (K_dx2), the shadow product of v is fused into its update (K_vnext).
@@ -47,10 +47,16 @@ constexpr int NBLK = 2 * 64 * 64;
 #ifndef VEC_NT
 #define VEC_NT 1
 #endif
-#ifndef SEG_BLOCKS
-#define SEG_BLOCKS 16
-#endif
-constexpr int SEG = SEG_BLOCKS;  // blocks per segment (work-group of the vector kernels)
+// blocks per segment (work-group of the vector kernels) of a column group of n blocks: a power of two, at most 16, and
+// few enough for 1,024 segments.  It depends on the group alone, so that a group's sums, and with them its iterates, do
+// not depend on the other groups of the plan.  With 16 blocks whatever the group, 1,024 blocks made 64 work-groups and
+// left three quarters of the CUs idle: FP64, 1,024 blocks: k_cocg_r 83 us against 29 with 1 block, k_cocg_px_odd 150
+// against 47; 1,461 blocks: k_dx2 348 against 117, k_even 160 against 85
+uint32_t segment_blocks(uint64_t n) {
+    uint32_t k = 16;
+    while (k > 1 && n < uint64_t(k) * 1024) k /= 2;
+    return k;
+}
 
 // per-column scalar fields, stored field-major: S[field * ncol + q]
 enum Field { RHO_RE, RHO_IM, ALPHA_RE, ALPHA_IM, THETA, TAU, ETAE_RE, ETAE_IM, ETAO_RE, ETAO_IM,
@@ -672,34 +678,56 @@ __global__ __launch_bounds__(256) void k_cocg_replace(T* __restrict__ rv, double
 // ------------------------------------------------------------------------------------------------
 __device__ __forceinline__ double& F(double* S, uint32_t ncol, int f, uint32_t q) { return S[uint64_t(f) * ncol + q]; }
 
-constexpr int FOLD_P = 8;  // waves folding the segments of one column group
+// The scalar kernels run one work-group of FOLD_T threads per column group and slice of 16 of its columns: thread
+// (j, part) adds every FOLD_P-th segment, so that 64 segments are in flight per column and the few groups of a plan
+// take four times as many CUs; threads tid < 16 then update column q = 64 c + 16 slice + tid.  (One work-group of 8
+// waves per group took 24 us for 4 groups of up to 600 segments, k_cocg_beta; this takes 10 us for twice the segments.)
+constexpr int FOLD_T = 1024, FOLD_P = FOLD_T / 16;
+#define FOLD_PROLOGUE \
+    uint32_t const c = blockIdx.x >> 2, slice = blockIdx.x & 3, q = 64 * c + 16 * slice + (threadIdx.x & 15); \
+    bool const owner = threadIdx.x < 16;
 
-// sums of the partial fields f[0..NC) of column group c over its segments: wave p adds segments
-// p, p + FOLD_P, ...; the waves' sums are then added in wave order (deterministic).  Valid in threads
-// tid < 64 (column j = tid).
-template <int NC>
-__device__ __forceinline__ void fold_group(double const* __restrict__ segpart, uint32_t const* __restrict__ col_seg,
-                                           uint32_t c, int const (&f)[NC], double (&tot)[NC]) {
-    __shared__ double sh[NC][FOLD_P][64];
-    int const tid = threadIdx.x, j = tid & 63, part = tid >> 6;
-    uint32_t const k0 = col_seg[c], k1 = col_seg[c + 1];
+// sums over k0 <= k < k1 of value(k, n), n < NC, at the thread's column (tid & 15), in an order that depends on
+// k1 - k0 only; valid in threads tid < 16
+template <int NC, typename Value>
+__device__ __forceinline__ void fold(uint32_t k0, uint32_t k1, double (&tot)[NC], Value&& value) {
+    __shared__ double sh[NC][FOLD_T / 64][16];
+    int const tid = threadIdx.x, jl = tid & 15, part = tid >> 4;
     double acc[NC];
 #pragma unroll
     for (int n = 0; n < NC; ++n) acc[n] = 0;
-    for (uint32_t k = k0 + part; k < k1; k += FOLD_P)
+#pragma unroll 4
+    for (uint32_t k = k0 + part; k < k1; k += FOLD_P) {
 #pragma unroll
-        for (int n = 0; n < NC; ++n) acc[n] += segpart[(uint64_t(k) * 3 + f[n]) * 64 + j];
+        for (int n = 0; n < NC; ++n) acc[n] += value(k, n);
+    }
 #pragma unroll
-    for (int n = 0; n < NC; ++n) sh[n][part][j] = acc[n];
+    for (int n = 0; n < NC; ++n) {   // the four parts of a wave, then the waves in order
+        acc[n] += __shfl_xor(acc[n], 16, 64);
+        acc[n] += __shfl_xor(acc[n], 32, 64);
+    }
+    if ((tid & 63) < 16) {
+#pragma unroll
+        for (int n = 0; n < NC; ++n) sh[n][tid >> 6][jl] = acc[n];
+    }
     __syncthreads();
-    if (tid < 64) {
+    if (tid < 16) {
 #pragma unroll
         for (int n = 0; n < NC; ++n) {
             double sum = 0;
-            for (int p = 0; p < FOLD_P; ++p) sum += sh[n][p][j];
+#pragma unroll
+            for (int w = 0; w < FOLD_T / 64; ++w) sum += sh[n][w][jl];
             tot[n] = sum;
         }
     }
+}
+
+// sums of the first NC partial fields of column group c over its segments
+template <int NC>
+__device__ __forceinline__ void fold_group(double const* __restrict__ segpart, uint32_t const* __restrict__ col_seg,
+                                           uint32_t c, uint32_t slice, double (&tot)[NC]) {
+    double const* src = segpart + slice * 16 + (threadIdx.x & 15);
+    fold<NC>(col_seg[c], col_seg[c + 1], tot, [&](uint32_t k, int n) { return src[(uint64_t(k) * 3 + n) * 64]; });
 }
 
 __device__ __forceinline__ void freeze_step(double* S, uint32_t ncol, uint32_t q) {
@@ -707,27 +735,23 @@ __device__ __forceinline__ void freeze_step(double* S, uint32_t ncol, uint32_t q
     for (int f = ETAE_RE; f <= BETA_IM; ++f) F(S, ncol, f, q) = 0;
 }
 
-// The scalar kernels run one work-group of 64 * FOLD_P threads per column group; threads tid < 64
-// update column q = 64 c + tid.
-
 // after k_init: |b|^2, (r0*, b); columns of inactive groups start as converged
-__global__ __launch_bounds__(64 * FOLD_P) void k_scalar_init(double* __restrict__ S, double const* __restrict__ segpart,
+__global__ __launch_bounds__(FOLD_T) void k_scalar_init(double* __restrict__ S, double const* __restrict__ segpart,
                                                           uint32_t const* __restrict__ col_seg,
                                                           uint8_t const* __restrict__ col_active, uint32_t ncol,
                                                           double tol_rel, double const* __restrict__ tol_abs) {
-    uint32_t const c = blockIdx.x, q = 64 * c + threadIdx.x;
+    FOLD_PROLOGUE
     if (!col_active[c]) {
-        if (threadIdx.x < 64) {
+        if (owner) {
             F(S, ncol, STATUS, q) = CONVERGED;
             F(S, ncol, MSTEP, q) = 0;
             freeze_step(S, ncol, q);
         }
         return;
     }
-    int const f[3] = {0, 1, 2};
     double t[3];
-    fold_group<3>(segpart, col_seg, c, f, t);
-    if (threadIdx.x >= 64) return;
+    fold_group<3>(segpart, col_seg, c, slice, t);
+    if (!owner) return;
     double const bn = sqrt(t[0]);
     F(S, ncol, BNORM, q) = bn;
     F(S, ncol, TAU, q) = bn;
@@ -743,15 +767,14 @@ __global__ __launch_bounds__(64 * FOLD_P) void k_scalar_init(double* __restrict_
 }
 
 // start of a step: alpha = rho / (r0*, v); a column that is no longer active gets zero coefficients
-__global__ __launch_bounds__(64 * FOLD_P) void k_scalar_alpha(double* __restrict__ S, double const* __restrict__ segpart,
+__global__ __launch_bounds__(FOLD_T) void k_scalar_alpha(double* __restrict__ S, double const* __restrict__ segpart,
                                                            uint32_t const* __restrict__ col_seg,
                                                            uint8_t const* __restrict__ col_active, uint32_t ncol) {
-    uint32_t const c = blockIdx.x, q = 64 * c + threadIdx.x;
+    FOLD_PROLOGUE
     if (!col_active[c]) return;
-    int const f[2] = {0, 1};
     double t[2];
-    fold_group<2>(segpart, col_seg, c, f, t);
-    if (threadIdx.x >= 64) return;
+    fold_group<2>(segpart, col_seg, c, slice, t);
+    if (!owner) return;
     if (F(S, ncol, STATUS, q) != ACTIVE) { freeze_step(S, ncol, q); return; }
     double const sr = t[0], si = t[1];
     double const den = sr * sr + si * si;
@@ -764,18 +787,15 @@ __global__ __launch_bounds__(64 * FOLD_P) void k_scalar_alpha(double* __restrict
 // after a w update: theta, c, tau, eta, the d coefficient, convergence; on odd half-steps also rho, beta.
 // Even half-steps write the E fields, odd ones the O fields (both are used by k_dx2).
 template <int ODD>
-__global__ __launch_bounds__(64 * FOLD_P) void k_scalar_theta(double* __restrict__ S, double const* __restrict__ segpart,
+__global__ __launch_bounds__(FOLD_T) void k_scalar_theta(double* __restrict__ S, double const* __restrict__ segpart,
                                                            uint32_t const* __restrict__ col_seg,
                                                            uint8_t const* __restrict__ col_active, uint32_t ncol) {
-    uint32_t const c = blockIdx.x, q = 64 * c + threadIdx.x;
+    FOLD_PROLOGUE
     if (!col_active[c]) return;
     constexpr int NC = ODD ? 3 : 1;
-    int f[NC];
     double t[NC];
-#pragma unroll
-    for (int n = 0; n < NC; ++n) f[n] = n;
-    fold_group<NC>(segpart, col_seg, c, f, t);
-    if (threadIdx.x >= 64) return;
+    fold_group<NC>(segpart, col_seg, c, slice, t);
+    if (!owner) return;
     int const FE = ODD ? ETAO_RE : ETAE_RE, FC = ODD ? CDO_RE : CDE_RE, FP = ODD ? ETAE_RE : ETAO_RE;
     if (F(S, ncol, STATUS, q) != ACTIVE) {
         F(S, ncol, FE, q) = 0; F(S, ncol, FE + 1, q) = 0;
@@ -826,13 +846,13 @@ __global__ __launch_bounds__(64 * FOLD_P) void k_scalar_theta(double* __restrict
 }
 
 // COCG: after k_cocg_init: |b|^2, (b, b); tolerance and status as k_scalar_init
-__global__ __launch_bounds__(64 * FOLD_P) void k_cocg_scalar_init(double* __restrict__ S, double const* __restrict__ segpart,
+__global__ __launch_bounds__(FOLD_T) void k_cocg_scalar_init(double* __restrict__ S, double const* __restrict__ segpart,
                                                                uint32_t const* __restrict__ col_seg,
                                                                uint8_t const* __restrict__ col_active, uint32_t ncol,
                                                                double tol_rel, double const* __restrict__ tol_abs) {
-    uint32_t const c = blockIdx.x, q = 64 * c + threadIdx.x;
+    FOLD_PROLOGUE
     if (!col_active[c]) {
-        if (threadIdx.x < 64) {
+        if (owner) {
             F(S, ncol, STATUS, q) = CONVERGED;
             F(S, ncol, MSTEP, q) = 0;
             F(S, ncol, RN, q) = 0;
@@ -840,10 +860,9 @@ __global__ __launch_bounds__(64 * FOLD_P) void k_cocg_scalar_init(double* __rest
         }
         return;
     }
-    int const f[3] = {0, 1, 2};
     double t[3];
-    fold_group<3>(segpart, col_seg, c, f, t);
-    if (threadIdx.x >= 64) return;
+    fold_group<3>(segpart, col_seg, c, slice, t);
+    if (!owner) return;
     double const bn = sqrt(t[0]);
     F(S, ncol, BNORM, q) = bn;
     F(S, ncol, RHO_RE, q) = t[1];
@@ -856,16 +875,29 @@ __global__ __launch_bounds__(64 * FOLD_P) void k_cocg_scalar_init(double* __rest
     F(S, ncol, RN, q) = (bn <= tol) ? 0.0 : 1.0;
 }
 
-// COCG: alpha = (r, r) / (p, A p)
-__global__ __launch_bounds__(64 * FOLD_P) void k_cocg_alpha(double* __restrict__ S, double const* __restrict__ segpart,
+// the per-block products (p, A p) of a group of at most this many blocks (16 per thread) are folded by the alpha kernel
+// itself; larger groups' are summed per segment first (k_fold_blocks)
+constexpr uint32_t DIRECT_BLOCKS = 16 * FOLD_P;
+
+// COCG: alpha = (r, r) / (p, A p), (p, A p) from the segment partials or, for a small group and unless bpart is null,
+// from the per-block products of the action
+__global__ __launch_bounds__(FOLD_T) void k_cocg_alpha(double* __restrict__ S, double const* __restrict__ segpart,
                                                          uint32_t const* __restrict__ col_seg,
-                                                         uint8_t const* __restrict__ col_active, uint32_t ncol) {
-    uint32_t const c = blockIdx.x, q = 64 * c + threadIdx.x;
+                                                         uint8_t const* __restrict__ col_active, uint32_t ncol,
+                                                         double const* __restrict__ bpart,
+                                                         uint32_t const* __restrict__ col_start,
+                                                         uint32_t const* __restrict__ col_blocks) {
+    FOLD_PROLOGUE
     if (!col_active[c]) return;
-    int const f[2] = {0, 1};
     double t[2];
-    fold_group<2>(segpart, col_seg, c, f, t);
-    if (threadIdx.x >= 64) return;
+    uint32_t const b0 = col_start[c], b1 = col_start[c + 1];
+    if (bpart && b1 - b0 <= DIRECT_BLOCKS) {
+        double const* src = bpart + slice * 16 + (threadIdx.x & 15);
+        fold<2>(b0, b1, t, [&](uint32_t k, int n) { return src[(uint64_t(col_blocks[k]) * 2 + n) * 64]; });
+    } else {
+        fold_group<2>(segpart, col_seg, c, slice, t);
+    }
+    if (!owner) return;
     if (F(S, ncol, STATUS, q) != ACTIVE) { freeze_step(S, ncol, q); return; }
     double const mr = t[0], mi = t[1], den = mr * mr + mi * mi;
     if (!(den > 0)) { F(S, ncol, STATUS, q) = BREAKDOWN; freeze_step(S, ncol, q); return; }
@@ -875,16 +907,15 @@ __global__ __launch_bounds__(64 * FOLD_P) void k_cocg_alpha(double* __restrict__
 }
 
 // COCG: after the r update: convergence on the recursive residual |r| <= tol; beta = (r', r') / (r, r)
-__global__ __launch_bounds__(64 * FOLD_P) void k_cocg_beta(double* __restrict__ S, double const* __restrict__ segpart,
+__global__ __launch_bounds__(FOLD_T) void k_cocg_beta(double* __restrict__ S, double const* __restrict__ segpart,
                                                         uint32_t const* __restrict__ col_seg,
                                                         uint8_t const* __restrict__ col_active, uint32_t ncol,
                                                         int save_alpha) {
-    uint32_t const c = blockIdx.x, q = 64 * c + threadIdx.x;
+    FOLD_PROLOGUE
     if (!col_active[c]) return;
-    int const f[3] = {0, 1, 2};
     double t[3];
-    fold_group<3>(segpart, col_seg, c, f, t);
-    if (threadIdx.x >= 64) return;
+    fold_group<3>(segpart, col_seg, c, slice, t);
+    if (!owner) return;
     if (save_alpha) {   // an even iteration: its x update is done by the next one (alpha 0 for stopped columns)
         F(S, ncol, APREV_RE, q) = F(S, ncol, ALPHA_RE, q);
         F(S, ncol, APREV_IM, q) = F(S, ncol, ALPHA_IM, q);
@@ -909,15 +940,14 @@ __global__ __launch_bounds__(64 * FOLD_P) void k_cocg_beta(double* __restrict__ 
 }
 
 // COCG after a residual replacement: rho = (r, r) of the replaced residual; convergence on its norm
-__global__ __launch_bounds__(64 * FOLD_P) void k_cocg_rho(double* __restrict__ S, double const* __restrict__ segpart,
+__global__ __launch_bounds__(FOLD_T) void k_cocg_rho(double* __restrict__ S, double const* __restrict__ segpart,
                                                        uint32_t const* __restrict__ col_seg,
                                                        uint8_t const* __restrict__ col_active, uint32_t ncol) {
-    uint32_t const c = blockIdx.x, q = 64 * c + threadIdx.x;
+    FOLD_PROLOGUE
     if (!col_active[c]) return;
-    int const f[3] = {0, 1, 2};
     double t[3];
-    fold_group<3>(segpart, col_seg, c, f, t);
-    if (threadIdx.x >= 64) return;
+    fold_group<3>(segpart, col_seg, c, slice, t);
+    if (!owner) return;
     if (F(S, ncol, STATUS, q) != ACTIVE) return;
     F(S, ncol, RHO_RE, q) = t[1];
     F(S, ncol, RHO_IM, q) = t[2];
@@ -925,15 +955,14 @@ __global__ __launch_bounds__(64 * FOLD_P) void k_cocg_rho(double* __restrict__ S
 }
 
 // residual norms of the active column groups (others keep their value)
-__global__ __launch_bounds__(64 * FOLD_P) void k_col_norm(double* __restrict__ res, double const* __restrict__ segpart,
+__global__ __launch_bounds__(FOLD_T) void k_col_norm(double* __restrict__ res, double const* __restrict__ segpart,
                                                        uint32_t const* __restrict__ col_seg,
                                                        uint8_t const* __restrict__ col_active) {
-    uint32_t const c = blockIdx.x;
+    FOLD_PROLOGUE
     if (!col_active[c]) return;
-    int const f[1] = {0};
     double t[1];
-    fold_group<1>(segpart, col_seg, c, f, t);
-    if (threadIdx.x < 64) res[64 * c + threadIdx.x] = sqrt(t[0]);
+    fold_group<1>(segpart, col_seg, c, slice, t);
+    if (owner) res[q] = sqrt(t[0]);
 }
 
 // x = 0 over whole blocks (a fill kernel rather than a memset, so that it may sit in a captured graph)
@@ -965,10 +994,12 @@ struct SolverState {
     // static structure
     std::vector<uint32_t> h_cstart, h_cb;   // blocks of column group c: h_cb[h_cstart[c] .. h_cstart[c+1])
     uint32_t* col_blocks = nullptr;
+    uint32_t* col_start = nullptr;          // [nCols+1] block range of each column group in col_blocks
     uint8_t* diag = nullptr;
     uint32_t* subset = nullptr;
-    // segments of <= SEG blocks of one column group, numbered once for the whole solve
+    // segments of a few blocks of one column group (segment_blocks), numbered once for the whole solve
     uint32_t nseg_all = 0;
+    uint32_t max_group_blocks = 0;          // blocks of the largest column group
     uint32_t* seg = nullptr;                // [nseg_all][3]
     uint32_t* col_seg = nullptr;            // [nCols+1] segment range of each column group
     std::vector<uint32_t> h_col_seg;
@@ -1068,9 +1099,12 @@ int setup(gfa_plan* plan, SolverState& st, std::string& err) {
     }
     std::vector<uint32_t> segs;
     st.h_col_seg.assign(1, 0);
+    st.max_group_blocks = 0;
     for (uint32_t c = 0; c < h.nCols; ++c) {
-        for (uint32_t b = st.h_cstart[c]; b < st.h_cstart[c + 1]; b += SEG) {
-            segs.push_back(c); segs.push_back(b); segs.push_back(std::min(st.h_cstart[c + 1], b + SEG));
+        uint32_t const b1 = st.h_cstart[c + 1], nb = b1 - st.h_cstart[c], n = segment_blocks(nb);
+        st.max_group_blocks = std::max(st.max_group_blocks, nb);
+        for (uint32_t b = st.h_cstart[c]; b < b1; b += n) {
+            segs.push_back(c); segs.push_back(b); segs.push_back(std::min(b1, b + n));
         }
         st.h_col_seg.push_back(uint32_t(segs.size() / 3));
     }
@@ -1079,6 +1113,7 @@ int setup(gfa_plan* plan, SolverState& st, std::string& err) {
     for (uint32_t c = 0; c < h.nCols; ++c) diag[h.subset[c]] = 1;
     int s;
     if ((s = walloc(st, st.col_blocks, h.nnzb, err))) return s;
+    if ((s = walloc(st, st.col_start, size_t(h.nCols) + 1, err))) return s;
     if ((s = walloc(st, st.diag, h.nnzb, err))) return s;
     if ((s = walloc(st, st.subset, h.nCols, err))) return s;
     if ((s = walloc(st, st.seg, size_t(st.nseg_all) * 3, err))) return s;
@@ -1088,6 +1123,7 @@ int setup(gfa_plan* plan, SolverState& st, std::string& err) {
     if ((s = walloc(st, st.act_items, h.nnzb * uint64_t(capi_dev(plan).head_words), err))) return s;
     if ((s = walloc(st, st.col_active, h.nCols, err))) return s;
     HIP_TRY(hipMemcpy(st.col_blocks, st.h_cb.data(), h.nnzb * 4, hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(st.col_start, st.h_cstart.data(), st.h_cstart.size() * 4, hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(st.diag, diag.data(), h.nnzb, hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(st.subset, h.subset.data(), size_t(h.nCols) * 4, hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(st.seg, segs.data(), segs.size() * 4, hipMemcpyHostToDevice));
@@ -1172,7 +1208,7 @@ template <typename T>
 int enqueue_step(gfa_plan* plan, SolverState& st, Vecs<T> const& V, uint64_t seed, hipStream_t s, std::string& err) {
     int const fp = sizeof(T) == 8 ? 64 : 32;
     SegArgs const g{st.act_seg, st.seg, st.col_blocks, st.segpart};
-    dim3 const gb(st.nseg), tb(256), gs(st.nCols), ts(64 * FOLD_P);
+    dim3 const gb(st.nseg), tb(256), gs(4 * st.nCols), ts(FOLD_T);
     hipLaunchKernelGGL(k_scalar_alpha, gs, ts, 0, s, st.S, st.segpart, st.col_seg, st.col_active, st.ncol);
     hipLaunchKernelGGL((k_even<T>), gb, tb, 0, s, V.un, V.u, V.v, V.w, V.Aeven, st.S, st.ncol, g);
     hipLaunchKernelGGL((k_scalar_theta<0>), gs, ts, 0, s, st.S, st.segpart, st.col_seg, st.col_active, st.ncol);
@@ -1272,7 +1308,7 @@ int tfqmr(gfa_plan* plan, SolverState& st, double const* rhs_y, double tol_rel, 
     int const fp = sizeof(T) == 8 ? 64 : 32;
     hipStream_t const s = st.stream;
     SegArgs const g{st.act_seg, st.seg, st.col_blocks, st.segpart};
-    dim3 const gs(st.nCols), ts(64 * FOLD_P);
+    dim3 const gs(4 * st.nCols), ts(FOLD_T);
     DevicePlan& dev = capi_dev(plan);
     ActiveScope scope(dev, st);
     if (st.nseg == 0) return 0;
@@ -1302,15 +1338,16 @@ int enqueue_cocg(gfa_plan* plan, SolverState& st, T* x, T* r, T* p0, T* p1, T* q
     T* const p = odd ? p1 : p0;
     int const fp = sizeof(T) == 8 ? 64 : 32;
     SegArgs const g{st.act_seg, st.seg, st.col_blocks, st.segpart};
-    dim3 const gb(st.nseg), tb(256), gs(st.nCols), ts(64 * FOLD_P);
+    dim3 const gb(st.nseg), tb(256), gs(4 * st.nCols), ts(FOLD_T);
     // (p, A p) from the action's epilogue when nothing is added to A p after the local kernel (no numax 6, 7
     // atoms, add-back on the vector ALUs), else from a pass over p and q
     DevicePlan const& dv = capi_dev(plan);
     bool const fused = dv.n_wide_blocks == 0 && dv.prj_engine[fp == 64 ? 0 : 1] == 0;
     if (int e = capi_action(plan, fp, q, p, s, err, ACTION_ALL, fused ? st.bpart : nullptr)) return e;
-    if (fused) hipLaunchKernelGGL(k_fold_blocks, gb, dim3(64), 0, s, st.bpart, g);
-    else hipLaunchKernelGGL((k_cocg_pq<T>), gb, tb, 0, s, p, q, g);
-    hipLaunchKernelGGL(k_cocg_alpha, gs, ts, 0, s, st.S, st.segpart, st.col_seg, st.col_active, st.ncol);
+    if (!fused) hipLaunchKernelGGL((k_cocg_pq<T>), gb, tb, 0, s, p, q, g);
+    else if (st.max_group_blocks > DIRECT_BLOCKS) hipLaunchKernelGGL(k_fold_blocks, gb, dim3(64), 0, s, st.bpart, g);
+    hipLaunchKernelGGL(k_cocg_alpha, gs, ts, 0, s, st.S, st.segpart, st.col_seg, st.col_active, st.ncol,
+                       fused ? st.bpart : nullptr, st.col_start, st.col_blocks);
     hipLaunchKernelGGL((k_cocg_r<T>), gb, tb, 0, s, r, q, st.S, st.ncol, g);
     hipLaunchKernelGGL(k_cocg_beta, gs, ts, 0, s, st.S, st.segpart, st.col_seg, st.col_active, st.ncol, odd ? 0 : 1);
     if (odd) hipLaunchKernelGGL((k_cocg_px_odd<T>), gb, tb, 0, s, x, p0, p1, r, st.S, st.ncol, g);
@@ -1340,7 +1377,7 @@ int cocg(gfa_plan* plan, SolverState& st, double const* rhs_y, double tol_rel, d
     {
         SegArgs const g{st.act_seg, st.seg, st.col_blocks, st.segpart};
         hipLaunchKernelGGL((k_cocg_init<T>), dim3(st.nseg), dim3(256), 0, s, r, p, rhs_y, st.diag, g);
-        hipLaunchKernelGGL(k_cocg_scalar_init, dim3(st.nCols), dim3(64 * FOLD_P), 0, s, st.S, st.segpart, st.col_seg,
+        hipLaunchKernelGGL(k_cocg_scalar_init, dim3(4 * st.nCols), dim3(FOLD_T), 0, s, st.S, st.segpart, st.col_seg,
                            st.col_active, st.ncol, tol_rel, tol_abs);
         if (f32) hipLaunchKernelGGL((k_zero_x<T>), dim3(st.nseg), dim3(256), 0, s, x, g);
         HIP_TRY(hipGetLastError());
@@ -1388,7 +1425,7 @@ int cocg(gfa_plan* plan, SolverState& st, double const* rhs_y, double tol_rel, d
         res.actions++;
         SegArgs const g2{st.act_seg, st.seg, st.col_blocks, st.segpart};
         hipLaunchKernelGGL((k_cocg_replace<T>), dim3(st.nseg), dim3(256), 0, s, r, y64, st.diag, g2);
-        hipLaunchKernelGGL(k_cocg_rho, dim3(st.nCols), dim3(64 * FOLD_P), 0, s, st.S, st.segpart, st.col_seg,
+        hipLaunchKernelGGL(k_cocg_rho, dim3(4 * st.nCols), dim3(FOLD_T), 0, s, st.S, st.segpart, st.col_seg,
                            st.col_active, st.ncol);
         HIP_TRY(hipGetLastError());
         return 0;
@@ -1428,7 +1465,7 @@ int residual(gfa_plan* plan, SolverState& st, int& actions, std::string& err) {
     actions++;
     SegArgs const g{st.act_seg, st.seg, st.col_blocks, st.segpart};
     hipLaunchKernelGGL((k_residual<double>), dim3(st.nseg), dim3(256), 0, s, st.y64, st.diag, g);
-    hipLaunchKernelGGL(k_col_norm, dim3(st.nCols), dim3(64 * FOLD_P), 0, s, st.res, st.segpart, st.col_seg,
+    hipLaunchKernelGGL(k_col_norm, dim3(4 * st.nCols), dim3(FOLD_T), 0, s, st.res, st.segpart, st.col_seg,
                        st.col_active);
     HIP_TRY(hipGetLastError());
     return 0;
@@ -1448,7 +1485,7 @@ uint64_t solve_bytes(gfa_plan* plan, int fp_bits, int method) {
     {
         std::vector<uint64_t> per(h.nCols, 0);
         for (uint64_t b = 0; b < nnzb; ++b) ++per[h.colindx[b]];
-        for (uint32_t c = 0; c < h.nCols; ++c) nseg += (per[c] + SEG - 1) / SEG;
+        for (uint32_t c = 0; c < h.nCols; ++c) nseg += (per[c] + segment_blocks(per[c]) - 1) / segment_blocks(per[c]);
     }
     uint64_t const vec64 = nnzb * NBLK * 8;
     uint64_t bytes = 2 * vec64;                          // x64, y64
@@ -1459,7 +1496,7 @@ uint64_t solve_bytes(gfa_plan* plan, int fp_bits, int method) {
         bytes += nnzb * 4 * uint64_t(wide ? 32 : 16);
     }
     bytes += nseg * (12 + 4) + nseg * 3 * 64 * 8;        // segments, active segments, segment partials
-    bytes += ncol * 8 * (NFIELDS + 2) + uint64_t(h.nCols) * 13;
+    bytes += ncol * 8 * (NFIELDS + 2) + uint64_t(h.nCols) * 17;
     int const m = method == 1 ? 1 : 0;
     uint64_t arena = uint64_t(fp_bits == 64 ? work_vectors<double>(m) * 2 : work_vectors<float>(m)) * (vec64 / 2);
     if (fp_bits == 32) arena = std::max(arena, uint64_t(work_vectors<double>(m)) * vec64);   // an FP64 fallback
