@@ -25,6 +25,7 @@
 #include <mutex>
 #include <cmath>
 #include <cstdio>
+#include <type_traits>
 
 namespace gfa {
 
@@ -619,6 +620,33 @@ __device__ __forceinline__ real_t nb_value(real_t const* __restrict__ b, int e, 
     return v;
 }
 
+// acc += the off-centre finite-difference weights applied to a window w of 4 (2 NH + 1) values centred at c, of the
+// 16th order if O16 (the centre weights of the three directions are applied together with the potential)
+template <typename real_t, int NH, int NW, bool O16>
+__device__ __forceinline__ void stencil(real_t& acc, LocalArgs<real_t> const& a, int d, real_t const (&w)[NW], int c) {
+    if constexpr (O16) {
+#pragma unroll
+        for (int m = 1; m <= 8; ++m) {
+            int const lo = c - m, hi = c + m;
+            acc += a.c16[d][m] * (w[lo < 0 ? 0 : lo] + w[hi >= NW ? NW - 1 : hi]);
+        }
+    } else {
+#pragma unroll
+        for (int m = 1; m <= 4; ++m) acc += a.c8[d][m] * (w[c - m] + w[c + m]);
+    }
+}
+
+// f(O16) with the order of direction d as a compile-time flag.  The branch (uniform) is taken once per pass: inside the
+// unrolled loops over the points it cost the 16th-order kernels half of their time (3,180 blocks FP32: k_plane 249 ->
+// 112 us, k_lines 242 -> 111)
+template <int NH, typename real_t, typename Fn>
+__device__ __forceinline__ void with_order(LocalArgs<real_t> const& a, int d, Fn&& f) {
+    if constexpr (NH == 2) {
+        if (a.nh[d] == 2) { f(std::true_type()); return; }
+    }
+    f(std::false_type());
+}
+
 // One work-group per (block, JW-column slice), 8*JW threads.  LDS holds the slice of the block
 // (xs) and the output accumulator (ys); passes: potential, kinetic x, y, z, SHO add-back, store.
 // In the kinetic passes a thread owns 4 lines (4 points each) of one (column, plane); neighbour
@@ -723,28 +751,17 @@ __global__ __launch_bounds__(8 * JW) void k_local(LocalArgs<real_t> a) {
                 }
             }
         }
+        // off-centre weights only: the centre weights are applied with the potential
+        with_order<NH>(a, d, [&](auto o16) {
 #pragma unroll
-        for (int r = 0; r < LB; ++r) {
+            for (int r = 0; r < LB; ++r)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                int const c = 4 * NH + q;
-                real_t t;
-                // off-centre weights only: the centre weights are applied with the potential
-                if (NH == 2 && a.nh[d] == 2) {
-                    t = a.c16[d][1] * (w[r][c - 1] + w[r][c + 1]);
-#pragma unroll
-                    for (int m = 2; m <= 8; ++m) {
-                        int const lo = c - m, hi = c + m;
-                        t += a.c16[d][m] * (w[r][lo < 0 ? 0 : lo] + w[r][hi >= NW ? NW - 1 : hi]);
-                    }
-                } else {
-                    t = a.c8[d][1] * (w[r][c - 1] + w[r][c + 1]);
-#pragma unroll
-                    for (int m = 2; m <= 4; ++m) t += a.c8[d][m] * (w[r][c - m] + w[r][c + m]);
+                for (int q = 0; q < 4; ++q) {
+                    real_t t = 0;
+                    stencil<real_t, NH, NW, decltype(o16)::value>(t, a, d, w[r], 4 * NH + q);
+                    ysp[(il0[r] + q * stride) * JW] += t;
                 }
-                ysp[(il0[r] + q * stride) * JW] += t;
-            }
-        }
+        });
         }  // line batches
     }
 
@@ -823,25 +840,9 @@ __device__ __forceinline__ void sho_add_regs(real_t (&out)[16], real_t const (*H
     });
 }
 
-// acc += the off-centre finite-difference weights applied to a window w of 4 (2 NH + 1) values centred at c
-// (the centre weights of the three directions are applied together with the potential)
-template <typename real_t, int NH, int NW>
-__device__ __forceinline__ void stencil(real_t& acc, LocalArgs<real_t> const& a, int d, real_t const (&w)[NW], int c) {
-    if (NH == 2 && a.nh[d] == 2) {
-#pragma unroll
-        for (int m = 1; m <= 8; ++m) {
-            int const lo = c - m, hi = c + m;
-            acc += a.c16[d][m] * (w[lo < 0 ? 0 : lo] + w[hi >= NW ? NW - 1 : hi]);
-        }
-    } else {
-#pragma unroll
-        for (int m = 1; m <= 4; ++m) acc += a.c8[d][m] * (w[c - m] + w[c + m]);
-    }
-}
-
 // z-direction stencil for the thread's plane ZQ: window positions z' = ZQ - 4 NH .. ZQ + 4 NH along z at every
 // (y, x); inside the block from LDS (own plane from registers), outside from the neighbour blocks
-template <typename real_t, int NH, bool IMG, int JW, int ZQ>
+template <typename real_t, int NH, bool IMG, int JW, int ZQ, bool O16>
 __device__ __forceinline__ void z_pass(LocalArgs<real_t> const& a, real_t (&acc)[16], real_t const (&own)[16],
                                        real_t const* __restrict__ xsp, real_t const* const (&nb)[2][NH],
                                        real_t const (&fr)[2][NH], real_t const (&fi)[2][NH], uint32_t boff_p, uint32_t boff_o) {
@@ -862,7 +863,7 @@ __device__ __forceinline__ void z_pass(LocalArgs<real_t> const& a, real_t (&acc)
                 w[m] = nb_value<real_t, IMG>(nb[1][kb], (zz * 16 + k) * 64, boff_p, boff_o, fr[1][kb], fi[1][kb]);
             }
         }
-        stencil<real_t, NH, NWZ>(acc[k], a, 2, w, 4 * NH);
+        stencil<real_t, NH, NWZ, O16>(acc[k], a, 2, w, 4 * NH);
     }
 }
 
@@ -916,6 +917,7 @@ __device__ __forceinline__ void plane_xy(LocalArgs<real_t> const& a, ItemHead<NH
         for (int sd = 0; sd < 2; ++sd)
 #pragma unroll
             for (int kk = 0; kk < NH; ++kk) nbz[sd][kk] = nb[sd][kk] + zqu * 16 * 64;
+        with_order<NH>(a, d, [&](auto o16) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             real_t w[NW];   // the line through this block and NH neighbour blocks on each side
@@ -933,9 +935,10 @@ __device__ __forceinline__ void plane_xy(LocalArgs<real_t> const& a, ItemHead<NH
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 int const k = (d == 0) ? (r * 4 + q) : (q * 4 + r);
-                stencil<real_t, NH, NW>(acc[k], a, d, w, 4 * NH + q);
+                stencil<real_t, NH, NW, decltype(o16)::value>(acc[k], a, d, w, 4 * NH + q);
             }
         }
+        });
     }
 }
 
@@ -1074,12 +1077,15 @@ __global__ __launch_bounds__(8 * JW) void k_plane(LocalArgs<real_t> a) {
         real_t const* nb[2][NH];
         real_t fr[2][NH], fi[2][NH];
         neighbours<real_t, NH, IMG>(a, 2, h, p, nb, fr, fi);
-        switch (zq) {
-            case 0: z_pass<real_t, NH, IMG, JW, 0>(a, acc, own, xsp, nb, fr, fi, boff_p, boff_o); break;
-            case 1: z_pass<real_t, NH, IMG, JW, 1>(a, acc, own, xsp, nb, fr, fi, boff_p, boff_o); break;
-            case 2: z_pass<real_t, NH, IMG, JW, 2>(a, acc, own, xsp, nb, fr, fi, boff_p, boff_o); break;
-            default: z_pass<real_t, NH, IMG, JW, 3>(a, acc, own, xsp, nb, fr, fi, boff_p, boff_o); break;
-        }
+        with_order<NH>(a, 2, [&](auto o16) {
+            constexpr bool O = decltype(o16)::value;
+            switch (zq) {
+                case 0: z_pass<real_t, NH, IMG, JW, 0, O>(a, acc, own, xsp, nb, fr, fi, boff_p, boff_o); break;
+                case 1: z_pass<real_t, NH, IMG, JW, 1, O>(a, acc, own, xsp, nb, fr, fi, boff_p, boff_o); break;
+                case 2: z_pass<real_t, NH, IMG, JW, 2, O>(a, acc, own, xsp, nb, fr, fi, boff_p, boff_o); break;
+                default: z_pass<real_t, NH, IMG, JW, 3, O>(a, acc, own, xsp, nb, fr, fi, boff_p, boff_o); break;
+            }
+        });
     }
 
     plane_finish<real_t, JW>(a, blk, h.w[IH_COL], h.w[IH_ADD0], h.w[IH_ADD1], slice, p, zq, jl, acc, xsp, xso, cs,
@@ -1132,6 +1138,7 @@ template <typename real_t, int NH>
 __device__ __forceinline__ void line_stencil(Lane<real_t> (&acc)[4], LocalArgs<real_t> const& a, int d,
                                              Lane<real_t> const (&own)[4], Lane<real_t> const (&w)[2][NH][4]) {
     constexpr int NW = 4 * (2 * NH + 1);
+    with_order<NH>(a, d, [&](auto o16) {
 #pragma unroll
     for (int c = 0; c < Lane<real_t>::n; ++c) {
         real_t win[NW];
@@ -1145,8 +1152,10 @@ __device__ __forceinline__ void line_stencil(Lane<real_t> (&acc)[4], LocalArgs<r
             }
         }
 #pragma unroll
-        for (int q = 0; q < 4; ++q) stencil<real_t, NH, NW>(acc[q].v[c], a, d, win, 4 * NH + q);
+        for (int q = 0; q < 4; ++q)
+            stencil<real_t, NH, NW, decltype(o16)::value>(acc[q].v[c], a, d, win, 4 * NH + q);
     }
+    });
 }
 
 // one z layer of sho_xline: the M = L - iz triangle of coefficients (iy + ix <= M, ix fastest) times
@@ -1207,9 +1216,8 @@ __device__ __forceinline__ void sho_xline(Lane<real_t> (&acc)[4], real_t const (
 }
 
 // the neighbour lines of direction d (NH blocks per side) of the lane's line starting at point i0, plane p and
-// first column j0, into w; a periodic-image neighbour (uniform over the work-group) gets its Bloch phase,
-// f x_p - (+/-) g x_other, which waits for its loads (image blocks are few)
-template <typename real_t, int NH, bool IMG>
+// first column j0, into w, without the Bloch phase of periodic images (phase_lines)
+template <typename real_t, int NH>
 __device__ __forceinline__ void load_lines(LocalArgs<real_t> const& a, int d, ItemHead<NH> const& h, int p, int i0,
                                            int j0, Lane<real_t> (&w)[2][NH][4]) {
     int const stride = (d == 0) ? 1 : ((d == 1) ? 4 : 16);
@@ -1224,33 +1232,39 @@ __device__ __forceinline__ void load_lines(LocalArgs<real_t> const& a, int d, It
 #pragma unroll
             for (int q = 0; q < 4; ++q) w[sd][k][q] = ldv(nb, q * stride * 64, off);
         }
-    if (IMG) {
-        uint32_t const offo = uint32_t((1 - p) * 4096 + i0 * 64 + j0) * sizeof(real_t);
+}
+
+// the Bloch phase of the periodic-image neighbours of direction d (uniform over the work-group) on their loaded lines,
+// f x_p - (+/-) g x_other: the same line of the other plane is in the lane LQ away, so nothing more is loaded
+template <typename real_t, int NH, int LQ>
+__device__ __forceinline__ void phase_lines(LocalArgs<real_t> const& a, int d, ItemHead<NH> const& h, int p,
+                                            Lane<real_t> (&w)[2][NH][4]) {
 #pragma unroll
-        for (int sd = 0; sd < 2; ++sd)
+    for (int sd = 0; sd < 2; ++sd)
 #pragma unroll
-            for (int k = 0; k < NH; ++k) {
-                int32_t const code = h.code(d, sd, k);
-                if (code <= -2) {
-                    real_t const* nb = a.x + uint64_t(-code - 2) * NBLK;
-                    real_t const fr = real_t(a.phase[d][sd][0]), fi = real_t(a.phase[d][sd][1]) * real_t(1 - 2 * p);
+        for (int k = 0; k < NH; ++k)
+            if (h.code(d, sd, k) <= -2) {
+                real_t const fr = real_t(a.phase[d][sd][0]), fi = real_t(a.phase[d][sd][1]) * real_t(1 - 2 * p);
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        Lane<real_t> const o = ldv(nb, q * stride * 64, offo);
+                for (int q = 0; q < 4; ++q)
 #pragma unroll
-                        for (int c = 0; c < Lane<real_t>::n; ++c) w[sd][k][q].v[c] = fr * w[sd][k][q].v[c] - fi * o.v[c];
+                    for (int c = 0; c < Lane<real_t>::n; ++c) {
+                        real_t const o = __shfl_xor(w[sd][k][q].v[c], LQ, 64);
+                        w[sd][k][q].v[c] = fr * w[sd][k][q].v[c] - fi * o;
                     }
-                }
             }
-    }
 }
 
 // PF: directions whose neighbour lines are issued before the first barrier (3: all; 2: x and y, z after the x
 // stencil; 1: x, then y after the x stencil and z after the y stencil) -- loads in flight against occupancy.
-// The FP64 shape with 16 columns and PF 2 needs 130 VGPRs on its own; it is held to 128 (4 waves per SIMD instead
-// of 3, one 8-byte spill), which makes it 6% faster; with PF 3 the same bound spills heavily and is not applied.
+// The FP64 shape with 16 columns and PF 2 is held to 128 VGPRs (4 waves per SIMD); with image phases the shuffles push
+// every 8th-order shape past 168, so those are held to 168 (3 waves, 5 spills; at 128 they spill 53).  Measured, FP64,
+// 16 columns, 2 directions: 512 blocks at a k-point 49 -> 32 us, 1,024 blocks 87 -> 57, 6,144 blocks 705 -> 368 against
+// loading the other plane's lines as well; 45,896 blocks without images 2,118 -> 2,050 us from loading the potential
+// before the barrier.  16th order: unbounded (184 VGPRs; held to 168, 11,474 blocks FP64 take 941 us instead of 829).
 template <typename real_t, int NH, bool IMG, int JW, int PF>
-__global__ __launch_bounds__((JW / Lane<real_t>::n) * 32, (sizeof(real_t) == 8 && JW == 16 && PF == 2) ? 4 : 1)
+__global__ __launch_bounds__((JW / Lane<real_t>::n) * 32,
+                             (sizeof(real_t) == 8 && JW == 16 && PF == 2 && !IMG) ? 4 : (IMG && NH == 1) ? 3 : 1)
 void k_lines(LocalArgs<real_t> a) {
     using L16 = Lane<real_t>;
     constexpr int CPL = L16::n, LQ = JW / CPL, T = LQ * 32;
@@ -1274,9 +1288,9 @@ void k_lines(LocalArgs<real_t> a) {
     int const ix0 = lb * 16 + la * 4, iy0 = lb * 16 + la, iz0 = lb * 4 + la;
 
     L16 wx[2][NH][4], wy[2][NH][4], wz[2][NH][4];   // neighbour lines per direction
-    load_lines<real_t, NH, IMG>(a, 0, h, p, ix0, j0, wx);
-    if constexpr (PF >= 2) load_lines<real_t, NH, IMG>(a, 1, h, p, iy0, j0, wy);
-    if constexpr (PF >= 3) load_lines<real_t, NH, IMG>(a, 2, h, p, iz0, j0, wz);
+    load_lines<real_t, NH>(a, 0, h, p, ix0, j0, wx);
+    if constexpr (PF >= 2) load_lines<real_t, NH>(a, 1, h, p, iy0, j0, wy);
+    if constexpr (PF >= 3) load_lines<real_t, NH>(a, 2, h, p, iz0, j0, wz);
     // own x-line, to registers and to the LDS copy of the slice
     L16 own[4];
     {
@@ -1286,6 +1300,11 @@ void k_lines(LocalArgs<real_t> a) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) st16(xs + (p * 64 + ix0 + q) * JW + jc, own[q]);
     }
+    // the potential on the x-line and the energy are loaded with the slice, before the barrier
+    int32_t const iv = int32_t(h.w[IH_VEFF]);
+    Lane<double> const V01 = ldv(a.V + uint64_t(iv >= 0 ? iv : 0) * 64, 0, uint32_t(ix0) * 8);
+    Lane<double> const V23 = ldv(a.V + uint64_t(iv >= 0 ? iv : 0) * 64, 2, uint32_t(ix0) * 8);
+    real_t const E_re = real_t(a.E_col[2 * h.w[IH_COL]]), E_im = real_t(a.E_col[2 * h.w[IH_COL] + 1]);
     __syncthreads();
 
     // ---- potential and x stencil on the x-line ----
@@ -1294,11 +1313,8 @@ void k_lines(LocalArgs<real_t> a) {
         L16 oth[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) oth[q] = ld16(xs + ((1 - p) * 64 + ix0 + q) * JW + jc);
-        int32_t const iv = int32_t(h.w[IH_VEFF]);
         real_t const vm = (iv >= 0) ? real_t(1) : real_t(0);
-        double const* Vb = a.V + uint64_t(iv >= 0 ? iv : 0) * 64 + ix0;
-        uint32_t const colE = h.w[IH_COL];
-        real_t const E_re = real_t(a.E_col[2 * colE]), E_im = real_t(a.E_col[2 * colE + 1]);
+        double const Vb[4] = {V01.v[0], V01.v[1], V23.v[0], V23.v[1]};
         real_t const Vim = E_im * real_t(1 - 2 * p);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -1306,10 +1322,11 @@ void k_lines(LocalArgs<real_t> a) {
 #pragma unroll
             for (int c = 0; c < CPL; ++c) acc[q].v[c] = dg * own[q].v[c] + Vim * oth[q].v[c];
         }
+        if (IMG) phase_lines<real_t, NH, LQ>(a, 0, h, p, wx);
         line_stencil<real_t, NH>(acc, a, 0, own, wx);
     }
-    if constexpr (PF < 2) load_lines<real_t, NH, IMG>(a, 1, h, p, iy0, j0, wy);
-    if constexpr (PF == 2) load_lines<real_t, NH, IMG>(a, 2, h, p, iz0, j0, wz);
+    if constexpr (PF < 2) load_lines<real_t, NH>(a, 1, h, p, iy0, j0, wy);
+    if constexpr (PF == 2) load_lines<real_t, NH>(a, 2, h, p, iz0, j0, wz);
 
     // ---- y stencil on the y-line, into ya ----
     {
@@ -1320,11 +1337,12 @@ void k_lines(LocalArgs<real_t> a) {
 #pragma unroll
             for (int c = 0; c < CPL; ++c) s[q].v[c] = 0;
         }
+        if (IMG) phase_lines<real_t, NH, LQ>(a, 1, h, p, wy);
         line_stencil<real_t, NH>(s, a, 1, o, wy);
 #pragma unroll
         for (int q = 0; q < 4; ++q) st16(ya + (p * 64 + iy0 + 4 * q) * JW + jc, s[q]);
     }
-    if constexpr (PF < 2) load_lines<real_t, NH, IMG>(a, 2, h, p, iz0, j0, wz);
+    if constexpr (PF < 2) load_lines<real_t, NH>(a, 2, h, p, iz0, j0, wz);
     __syncthreads();
     // ---- z stencil on the z-line, added into ya ----
     {
@@ -1334,6 +1352,7 @@ void k_lines(LocalArgs<real_t> a) {
             o[q] = ld16(xs + (p * 64 + iz0 + 16 * q) * JW + jc);
             s[q] = ld16(ya + (p * 64 + iz0 + 16 * q) * JW + jc);
         }
+        if (IMG) phase_lines<real_t, NH, LQ>(a, 2, h, p, wz);
         line_stencil<real_t, NH>(s, a, 2, o, wz);
 #pragma unroll
         for (int q = 0; q < 4; ++q) st16(ya + (p * 64 + iz0 + 16 * q) * JW + jc, s[q]);
