@@ -79,9 +79,9 @@ __device__ __forceinline__ void hermite_1d(real_t (*H)[3][4], float (*xi2)[4], i
 }
 
 // The Hermite functions of every (atom image, target row) pair that the projection and the add-back use, computed
-// once per plan with hermite_1d itself (so the values are those the kernels computed on the fly before):
-// htab[slot][8][3][4] (FP64, numax <= 7) and xtab[slot][3][4] = xi^2 (float).
-__global__ __launch_bounds__(64) void k_hermite_table(double* __restrict__ htab, float* __restrict__ xtab,
+// once per plan with hermite_1d itself: htab[slot][8][3][4] (FP64, numax <= 7), and in smask[slot] the points (bit
+// (z * 4 + y) * 4 + x) inside the projection sphere, tested in float from xi^2.
+__global__ __launch_bounds__(64) void k_hermite_table(double* __restrict__ htab, uint64_t* __restrict__ smask,
                                                       uint32_t const* __restrict__ slot_img,
                                                       uint32_t const* __restrict__ slot_row,
                                                       double const* __restrict__ image_pos,
@@ -90,29 +90,27 @@ __global__ __launch_bounds__(64) void k_hermite_table(double* __restrict__ htab,
                                                       double hz, double rproj) {
     uint32_t const sl = blockIdx.x;
     int const t = threadIdx.x;
-    if (t >= 12) return;
     uint32_t const img = slot_img[sl], row = slot_row[sl];
     double const hgrid[4] = {hx, hy, hz, rproj};
-    hermite_1d<double>(reinterpret_cast<double (*)[3][4]>(htab + size_t(sl) * 96),
-                       reinterpret_cast<float (*)[4]>(xtab + size_t(sl) * 12), t, image_lmax[img],
-                       image_pos + 4 * size_t(img), row_pos + 4 * size_t(row), hgrid);
+    __shared__ float xi2[3][4];
+    if (t < 12)
+        hermite_1d<double>(reinterpret_cast<double (*)[3][4]>(htab + size_t(sl) * 96), xi2, t, image_lmax[img],
+                           image_pos + 4 * size_t(img), row_pos + 4 * size_t(row), hgrid);
+    __syncthreads();
+    float const R2 = float(rproj * rproj);
+    float const d2z = xi2[2][t >> 4] - R2;
+    float const d2yz = xi2[1][(t >> 2) & 3] + d2z;
+    float const d2 = xi2[0][t & 3] + d2yz;
+    uint64_t const in = __ballot((d2z < 0) && (d2yz < 0) && (d2 < 0));
+    if (t == 0) smask[sl] = in;
 }
 
-// stage the table entry of `slot` into the LDS arrays H[L+1][3][4] (real_t) and xi2[3][4]; no barrier
+// stage the table entry of `slot` into the LDS array H[L+1][3][4] (real_t); no barrier
 template <typename real_t>
-__device__ __forceinline__ void stage_hermite(real_t (*H)[3][4], float (*xi2)[4], double const* __restrict__ htab,
-                                              float const* __restrict__ xtab, uint32_t slot, int L, int tid, int T) {
+__device__ __forceinline__ void stage_hermite(real_t (*H)[3][4], double const* __restrict__ htab, uint32_t slot, int L,
+                                              int tid, int T) {
     double const* src = htab + size_t(slot) * 96;
     for (int e = tid; e < (L + 1) * 12; e += T) H[e / 12][(e % 12) / 4][e % 4] = real_t(src[e]);
-    if (tid < 12) xi2[tid / 4][tid % 4] = xtab[size_t(slot) * 12 + tid];
-}
-
-// is point (y, x) of z plane zq inside the projection sphere (the 3D mask evaluated in float from xi^2)
-__device__ __forceinline__ bool sho_inside(float const (*xi2)[4], float R2, int zq, int y, int xx) {
-    float const d2z = xi2[2][zq] - R2;
-    float const d2yz = xi2[1][y] + d2z;
-    float const d2 = xi2[0][xx] + d2yz;
-    return (d2z < 0) && (d2yz < 0) && (d2 < 0);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -125,9 +123,8 @@ __global__ __launch_bounds__(128) void k_sho_project(
     uint32_t const* __restrict__ prj_blocks, uint32_t const* __restrict__ rowindx,
     float const* __restrict__ row_pos, double const* __restrict__ image_pos, double hx, double hy, double hz,
     double rproj, uint8_t const* __restrict__ col_active, double const* __restrict__ htab,
-    float const* __restrict__ xtab, uint32_t const* __restrict__ prj_slot) {
+    uint64_t const* __restrict__ smask, uint32_t const* __restrict__ prj_slot) {
     __shared__ real_t H[L + 1][3][4];
-    __shared__ float xi2[3][4];
     uint32_t const ich = bucket[blockIdx.x];
     ProjChunk const ch = chunks[ich];
     if (col_active && !col_active[ch.col]) return;  // a retired column group
@@ -137,17 +134,18 @@ __global__ __launch_bounds__(128) void k_sho_project(
     real_t czyx[n3];
 #pragma unroll
     for (int s = 0; s < n3; ++s) czyx[s] = 0;
-    float const R2 = float(rproj * rproj);
+    (void)rproj;
     for (uint32_t b = ch.begin; b < ch.end; ++b) {
         uint32_t const inzb = prj_blocks[b];
+        uint64_t const in = smask[prj_slot[b]];   // uniform
         __syncthreads();
-        stage_hermite<real_t>(H, xi2, htab, xtab, prj_slot[b], L, tid, 128);
+        stage_hermite<real_t>(H, htab, prj_slot[b], L, tid, 128);
         __syncthreads();
         real_t const* xb = x + size_t(inzb) * NBLK + p * 4096 + j;
 #pragma unroll
         for (int z = 0; z < 4; ++z) {
-            float const d2z = xi2[2][z] - R2;
-            if (d2z < 0) {
+            uint32_t const inz = uint32_t(in >> (16 * z)) & 0xffff;
+            if (inz) {
                 // the 16 points of the plane are loaded together (unconditionally, all in the block) and the
                 // sphere mask is applied as a select, so the loads are in flight at once
                 real_t v[16];
@@ -158,15 +156,14 @@ __global__ __launch_bounds__(128) void k_sho_project(
                 for (int k = 0; k < n2; ++k) byx[k] = 0;
 #pragma unroll
                 for (int y = 0; y < 4; ++y) {
-                    float const d2yz = xi2[1][y] + d2z;
-                    if (d2yz < 0) {
+                    uint32_t const iny = (inz >> (4 * y)) & 15;
+                    if (iny) {
                         real_t ax[L + 1];
 #pragma unroll
                         for (int k = 0; k <= L; ++k) ax[k] = 0;
 #pragma unroll
                         for (int xx = 0; xx < 4; ++xx) {
-                            float const d2 = xi2[0][xx] + d2yz;
-                            real_t const ps = (d2 < 0) ? v[y * 4 + xx] : real_t(0);
+                            real_t const ps = ((iny >> xx) & 1) ? v[y * 4 + xx] : real_t(0);
 #pragma unroll
                             for (int k = 0; k <= L; ++k) ax[k] += ps * H[k][0][xx];
                         }
@@ -227,13 +224,12 @@ template <typename real_t, int L>
 __global__ __launch_bounds__(256) void k_sho_project_mfma(
     real_t* __restrict__ partial, real_t const* __restrict__ x, ProjChunk const* __restrict__ chunks,
     uint32_t const* __restrict__ bucket, uint32_t const* __restrict__ chunk_coef,
-    uint32_t const* __restrict__ prj_blocks, double rproj, uint8_t const* __restrict__ col_active,
-    double const* __restrict__ htab, float const* __restrict__ xtab, uint32_t const* __restrict__ prj_slot) {
+    uint32_t const* __restrict__ prj_blocks, uint8_t const* __restrict__ col_active,
+    double const* __restrict__ htab, uint64_t const* __restrict__ smask, uint32_t const* __restrict__ prj_slot) {
     using acc_t = typename Mfma<real_t>::acc_t;
     constexpr int NC = Sho<L>::n3, MT = (NC + 15) / 16, NCP = 16 * MT;
     __shared__ real_t P[64 * NCP];           // [point][coefficient], zero beyond NC and outside the sphere
     __shared__ real_t H[L + 1][3][4];
-    __shared__ float xi2[3][4];
     __shared__ uint16_t sxyz[NCP];           // coefficient s -> ix | iy << 4 | iz << 8
     uint32_t const ich = bucket[blockIdx.x];
     ProjChunk const ch = chunks[ich];
@@ -246,7 +242,6 @@ __global__ __launch_bounds__(256) void k_sho_project_mfma(
                 for (int ix = 0; ix <= L - iz - iy; ++ix) sxyz[s++] = uint16_t(ix | (iy << 4) | (iz << 8));
         for (; s < NCP; ++s) sxyz[s] = 0xFFFF;
     }
-    float const R2 = float(rproj * rproj);
     acc_t acc[MT][2];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
@@ -264,14 +259,15 @@ __global__ __launch_bounds__(256) void k_sho_project_mfma(
             bv[ks][1] = xb[(ks * 4 + kl) * 64 + 16];
         }
         __syncthreads();   // P of the previous block is no longer read
-        stage_hermite<real_t>(H, xi2, htab, xtab, prj_slot[b], L, tid, 256);
+        uint64_t const in = smask[prj_slot[b]];   // uniform
+        stage_hermite<real_t>(H, htab, prj_slot[b], L, tid, 256);
         __syncthreads();
         for (int e = tid; e < 64 * NCP; e += 256) {
             int const i = e / NCP, s = e % NCP;
             int const xx = i & 3, yy = (i >> 2) & 3, zz = i >> 4;
             uint16_t const c = sxyz[s];
             real_t v = 0;
-            if (c != 0xFFFF && sho_inside(xi2, R2, zz, yy, xx))
+            if (c != 0xFFFF && ((in >> i) & 1))
                 v = H[c & 15][0][xx] * H[(c >> 4) & 15][1][yy] * H[c >> 8][2][zz];
             P[e] = v;
         }
@@ -499,7 +495,7 @@ struct LocalArgs {
     uint32_t per_xcd;        // work-items per XCD in the XCD-contiguous mapping
     double const* E_col;     // [nCols][2] energy of each column group
     double const* htab;      // Hermite functions per (image, row) slot
-    float const* xtab;
+    uint64_t const* smask;   // points inside the projection sphere per slot
     double* dot;             // if set: [nnzb][re, im][64] bilinear products sum_i x[b][i][j] y[b][i][j] per block
     int add_local;           // 1: the local kernel adds the numax <= 5 images; 0: k_sho_add_mfma adds them after it
     real_t c8[3][5];         // 8th-order weights per direction
@@ -510,23 +506,12 @@ struct LocalArgs {
     double hgrid[4];
 };
 
-// one z layer iz of the contraction in sho_plane: the M = L - iz triangle of coefficients (iy + ix <= M, ix
-// fastest) times H_z[iz](zq), accumulated into c2[iy][ix] (triangular with rows of the full L triangle)
-template <typename real_t, int L, int M>
-__device__ __forceinline__ void sho_z_layer(real_t (&c2)[((L + 1) * (L + 2)) / 2], real_t const* __restrict__ src,
-                                            size_t dstride, real_t hz) {
-    int t = 0;
-#pragma unroll
-    for (int iy = 0; iy <= M; ++iy)
-#pragma unroll
-        for (int ix = 0; ix <= M - iy; ++ix, ++t) c2[(iy * (2 * L + 3 - iy)) / 2 + ix] += src[size_t(t) * dstride] * hz;
-}
-
 // sum over the SHO coefficients c[iz][iy][ix] (ix fastest, iz + iy + ix <= L) of one atom image at the 16
 // points (y, x) of the z plane zq, v(y, x) = sum c H_x[ix](x) H_y[iy](y) H_z[iz](zq), handed to out(y, x, v).
 // Contracted z first (one value H_z[iz](zq) per thread), then y and x row by row: (L+1)(L+2)(L+3)/6 +
-// 4 (L+1)(L+2)/2 + 16 (L+1) FMAs.  The z layers run in a rolled loop, so at most one layer of coefficients is
-// loaded ahead; ROLL keeps the row loop rolled as well (out must then accept a run-time row y).
+// 4 (L+1)(L+2)/2 + 16 (L+1) FMAs.  All loops are unrolled, with a scheduling barrier after every z layer so that at
+// most one layer of coefficients is loaded ahead (rolled layers with a run-time size cost a copy of all sums per
+// layer: more moves than FMAs); ROLL keeps the row loop rolled (out must then accept a run-time row y).
 // dsrc points to coefficient 0 of this thread's (plane, column); consecutive coefficients are dstride apart.
 template <typename real_t, int L, bool ROLL, typename Out>
 __device__ __forceinline__ void sho_plane(real_t const (*H)[3][4], real_t const* __restrict__ dsrc, size_t dstride,
@@ -535,21 +520,16 @@ __device__ __forceinline__ void sho_plane(real_t const (*H)[3][4], real_t const*
     real_t c2[n2];   // [iy][ix] triangular, row iy starts at iy (2L + 3 - iy) / 2
 #pragma unroll
     for (int k = 0; k < n2; ++k) c2[k] = 0;
-    real_t const* src = dsrc;
-#pragma unroll 1
+    int t = 0;
+#pragma unroll
     for (int iz = 0; iz <= L; ++iz) {
         real_t const hz = H[iz][2][zq];
-        switch (L - iz) {
-            case 0: sho_z_layer<real_t, L, 0>(c2, src, dstride, hz); break;
-            case 1: if constexpr (L >= 1) sho_z_layer<real_t, L, 1>(c2, src, dstride, hz); break;
-            case 2: if constexpr (L >= 2) sho_z_layer<real_t, L, 2>(c2, src, dstride, hz); break;
-            case 3: if constexpr (L >= 3) sho_z_layer<real_t, L, 3>(c2, src, dstride, hz); break;
-            case 4: if constexpr (L >= 4) sho_z_layer<real_t, L, 4>(c2, src, dstride, hz); break;
-            case 5: if constexpr (L >= 5) sho_z_layer<real_t, L, 5>(c2, src, dstride, hz); break;
-            case 6: if constexpr (L >= 6) sho_z_layer<real_t, L, 6>(c2, src, dstride, hz); break;
-            default: if constexpr (L >= 7) sho_z_layer<real_t, L, 7>(c2, src, dstride, hz); break;
-        }
-        src += size_t(((L - iz + 1) * (L - iz + 2)) / 2) * dstride;
+#pragma unroll
+        for (int iy = 0; iy <= L - iz; ++iy)
+#pragma unroll
+            for (int ix = 0; ix <= L - iz - iy; ++ix, ++t)
+                c2[(iy * (2 * L + 3 - iy)) / 2 + ix] += dsrc[size_t(t) * dstride] * hz;
+        __builtin_amdgcn_sched_barrier(0);
     }
     auto row = [&](int y) {
         real_t by[L + 1];
@@ -578,33 +558,104 @@ __device__ __forceinline__ void sho_plane(real_t const (*H)[3][4], real_t const*
     }
 }
 
-// sho_plane for a run-time numax L <= LMAX (LMAX <= 7)
-template <typename real_t, int LMAX, bool ROLL, typename Out>
+// sho_plane for a run-time numax LMIN <= L <= LMAX
+template <typename real_t, int LMIN, int LMAX, bool ROLL, typename Out>
 __device__ __forceinline__ void sho_plane_any(real_t const (*H)[3][4], real_t const* __restrict__ dsrc, size_t dstride,
                                               int zq, int L, Out&& out) {
-    switch (L) {
-        case 0: sho_plane<real_t, 0, ROLL>(H, dsrc, dstride, zq, out); break;
-        case 1: sho_plane<real_t, 1, ROLL>(H, dsrc, dstride, zq, out); break;
-        case 2: sho_plane<real_t, 2, ROLL>(H, dsrc, dstride, zq, out); break;
-        case 3: sho_plane<real_t, 3, ROLL>(H, dsrc, dstride, zq, out); break;
-        case 4: sho_plane<real_t, 4, ROLL>(H, dsrc, dstride, zq, out); break;
-        case 5: sho_plane<real_t, 5, ROLL>(H, dsrc, dstride, zq, out); break;
-        case 6: if constexpr (LMAX >= 6) sho_plane<real_t, 6, ROLL>(H, dsrc, dstride, zq, out); break;
-        default: if constexpr (LMAX >= 7) sho_plane<real_t, 7, ROLL>(H, dsrc, dstride, zq, out); break;
+    if constexpr (LMIN < LMAX) {
+        if (L == LMIN) sho_plane<real_t, LMIN, ROLL>(H, dsrc, dstride, zq, out);
+        else sho_plane_any<real_t, LMIN + 1, LMAX, ROLL>(H, dsrc, dstride, zq, L, out);
+    } else {
+        sho_plane<real_t, LMAX, ROLL>(H, dsrc, dstride, zq, out);
     }
 }
 
-
-// SHO add-back of one atom image (numax L <= LMAX) into this thread's z plane zq of an accumulator in memory
-// (LDS or global) whose points are ostride apart: ys[(zq*16 + y*4 + x) * ostride]
-template <typename real_t, int LMAX>
-__device__ __forceinline__ void sho_add_atom(real_t* __restrict__ ys, int ostride, real_t const (*H)[3][4],
-                                             float const (*xi2)[4], float R2, real_t const* __restrict__ dsrc,
-                                             size_t dstride, int zq, int L) {
-    sho_plane_any<real_t, LMAX, true>(H, dsrc, dstride, zq, L, [&](int y, int xx, real_t v) {
+// SHO add-back of one atom image (numax L <= 5) into this thread's z plane zq of an accumulator in LDS whose points are
+// ostride apart: ys[(zq*16 + y*4 + x) * ostride]; in: the points inside the projection sphere
+template <typename real_t>
+__device__ __forceinline__ void sho_add_atom(real_t* __restrict__ ys, int ostride, real_t const (*H)[3][4], uint64_t in,
+                                             real_t const* __restrict__ dsrc, size_t dstride, int zq, int L) {
+    sho_plane_any<real_t, 0, 5, true>(H, dsrc, dstride, zq, L, [&](int y, int xx, real_t v) {
         real_t& o = ys[(zq * 16 + y * 4 + xx) * ostride];
-        o += sho_inside(xi2, R2, zq, y, xx) ? v : real_t(0);
+        o += ((in >> (zq * 16 + y * 4 + xx)) & 1) ? v : real_t(0);
     });
+}
+
+// SHO add-back of one atom image (LMIN <= numax <= LMAX) into 16 register accumulators (z plane zq of one column and
+// plane); in: the plane's points inside the projection sphere (16 bits)
+template <typename real_t, int LMIN, int LMAX>
+__device__ __forceinline__ void sho_add_regs(real_t (&out)[16], real_t const (*H)[3][4], uint32_t in,
+                                             real_t const* __restrict__ dsrc, size_t dstride, int zq, int L) {
+    sho_plane_any<real_t, LMIN, LMAX, false>(H, dsrc, dstride, zq, L, [&](int y, int xx, real_t v) {
+        out[y * 4 + xx] += ((in >> (y * 4 + xx)) & 1) ? v : real_t(0);
+    });
+}
+
+// The images of a block's add list are taken in batches whose coefficients fit a buffer of CAP rows in LDS, so that a
+// work-group pays one round trip to memory and two barriers per batch: with numax 2 four images, numax 3 two, numax 4
+// and 5 one at a time.
+constexpr int BATCH = 4;
+template <typename real_t>
+struct BatchHermite { real_t H[BATCH][6][3][4]; };
+
+// stages the next images (numax <= 5) of the add list from entry b on (column group col, columns from c0 on) into cs
+// [coefficient][plane][JW] and bh, for all T threads of the work-group (it contains two barriers, and the buffers are
+// free before the first); returns the entry after the batch.  The k-th image of the batch with numax L <= 5 has its
+// coefficients behind those of the images before it.
+template <typename real_t, int JW, int T, int CAP>
+__device__ __forceinline__ uint32_t stage_batch(LocalArgs<real_t> const& a, uint32_t b, uint32_t b1, uint32_t col,
+                                                int c0, real_t* cs, BatchHermite<real_t>& bh) {
+    typedef real_t __attribute__((ext_vector_type(16 / sizeof(real_t)))) vec_t;
+    constexpr int VE = 16 / sizeof(real_t), VPR = JW / VE;   // 16-byte vectors per row
+    constexpr int NV = (2 * CAP * VPR + T - 1) / T;          // of them per thread in a full buffer
+    int const tid = threadIdx.x;
+    uint32_t slot[BATCH], coef[BATCH], row0[BATCH + 1];      // uniform; rows: 2 per coefficient
+    int n = 0;
+    row0[0] = 0;
+#pragma unroll
+    for (int q = 0; q < BATCH; ++q) {
+        bool take = false;
+        uint32_t nc = 0;
+        slot[q] = q ? slot[0] : 0;   // entries beyond the batch are loaded like the first, and not used
+        coef[q] = q ? coef[0] : 0;
+        for (; b < b1; ++b) {
+            AddEntry const e = a.add_entry[b];
+            if (e.L > 5) continue;   // added by k_sho_add_wide
+            nc = ((e.L + 1) * (e.L + 2) * (e.L + 3)) / 6;
+            take = row0[q] + 2 * nc <= 2 * CAP;
+            if (take) { slot[q] = e.slot; coef[q] = e.coef0; }
+            break;
+        }
+        row0[q + 1] = row0[q] + (take ? 2 * nc : 0);
+        if (take) { ++b; ++n; }
+    }
+    uint32_t const rows = row0[BATCH];
+    vec_t t[NV];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+        uint32_t const v = k * T + tid, row = v / VPR, cv = v % VPR;   // row = coefficient * 2 + plane
+        uint32_t base = coef[0], r0 = 0;
+#pragma unroll
+        for (int q = 1; q < BATCH; ++q)
+            if (row >= row0[q] && row0[q + 1] > row0[q]) { base = coef[q]; r0 = row0[q]; }
+        uint32_t const r = (row < rows) ? row - r0 : 0;   // beyond the batch: a row of it again, not stored
+        t[k] = *reinterpret_cast<vec_t const*>(a.dcoef + (size_t(base + (r >> 1)) * a.nCols + col) * 128 + (r & 1) * 64 +
+                                               c0 + cv * VE);
+    }
+    real_t h[BATCH];
+#pragma unroll
+    for (int q = 0; q < BATCH; ++q) h[q] = real_t(a.htab[size_t(slot[q]) * 96 + (tid < 72 ? tid : 0)]);
+    __syncthreads();   // the buffers are no longer read
+#pragma unroll
+    for (int q = 0; q < BATCH; ++q)
+        if (q < n && tid < 72) bh.H[q][tid / 12][(tid % 12) / 4][tid % 4] = h[q];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+        uint32_t const v = k * T + tid, row = v / VPR, cv = v % VPR;
+        if (row < rows) *reinterpret_cast<vec_t*>(cs + row * JW + cv * VE) = t[k];
+    }
+    __syncthreads();
+    return b;
 }
 
 // value of a neighbour block at point e (a compile-time element offset from the uniform pointer b) and byte
@@ -658,8 +709,7 @@ __global__ __launch_bounds__(8 * JW) void k_local(LocalArgs<real_t> a) {
     constexpr int NSLICE = 64 / JW;
     __shared__ real_t xs[2 * 64 * JW];
     __shared__ real_t ys[2 * 64 * JW];
-    __shared__ real_t H[8][3][4];
-    __shared__ float xi2[3][4];
+    __shared__ real_t H[6][3][4];
 
     uint64_t lin = blockIdx.x;
     if (a.per_xcd) lin = uint64_t(blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
@@ -770,7 +820,6 @@ __global__ __launch_bounds__(8 * JW) void k_local(LocalArgs<real_t> a) {
     uint32_t const b0 = h.w[IH_ADD0], b1 = h.w[IH_ADD1];
     if (a.add_local && b1 > b0) {
         uint32_t const col = h.w[IH_COL];
-        float const R2 = float(a.hgrid[3] * a.hgrid[3]);
         int const zq = lg;  // threads (jl, p, zq) own the z plane zq
         real_t* cs = xs;    // [nc][2][JW]
         for (uint32_t b = b0; b < b1; ++b) {
@@ -779,7 +828,7 @@ __global__ __launch_bounds__(8 * JW) void k_local(LocalArgs<real_t> a) {
             if (L > 5) continue;  // done by k_sho_add_wide
             int const nc = ((L + 1) * (L + 2) * (L + 3)) / 6;
             __syncthreads();
-            stage_hermite<real_t>(H, xi2, a.htab, a.xtab, e.slot, L, tid, T);
+            stage_hermite<real_t>(H, a.htab, e.slot, L, tid, T);
             {
                 real_t const* src = a.dcoef + (size_t(e.coef0) * a.nCols + col) * 128 + slice * JW;
                 for (int v = tid; v < 2 * nc * VPR; v += T) {
@@ -789,7 +838,7 @@ __global__ __launch_bounds__(8 * JW) void k_local(LocalArgs<real_t> a) {
                 }
             }
             __syncthreads();
-            sho_add_atom<real_t, 5>(ysp, JW, H, xi2, R2, cs + p * JW + jl, 2 * JW, zq, L);
+            sho_add_atom<real_t>(ysp, JW, H, a.smask[e.slot], cs + p * JW + jl, 2 * JW, zq, L);
         }
     }
     __syncthreads();
@@ -830,15 +879,6 @@ __global__ __launch_bounds__(8 * JW) void k_local(LocalArgs<real_t> a) {
     }
 }
 
-
-// SHO add-back of one atom image (numax <= 5) into 16 register accumulators (z plane zq of one column and plane)
-template <typename real_t>
-__device__ __forceinline__ void sho_add_regs(real_t (&out)[16], real_t const (*H)[3][4], float const (*xi2)[4],
-                                             float R2, real_t const* __restrict__ dsrc, size_t dstride, int zq, int L) {
-    sho_plane_any<real_t, 5, false>(H, dsrc, dstride, zq, L, [&](int y, int xx, real_t v) {
-        out[y * 4 + xx] += sho_inside(xi2, R2, zq, y, xx) ? v : real_t(0);
-    });
-}
 
 // z-direction stencil for the thread's plane ZQ: window positions z' = ZQ - 4 NH .. ZQ + 4 NH along z at every
 // (y, x); inside the block from LDS (own plane from registers), outside from the neighbour blocks
@@ -953,30 +993,22 @@ template <typename real_t, int JW>
 __device__ __forceinline__ void plane_finish(LocalArgs<real_t> const& a, uint64_t blk, uint32_t col, uint32_t b0,
                                              uint32_t b1, int slice, int p, int zq, int jl, real_t (&acc)[16],
                                              real_t const* xsp, real_t const* xso, real_t* cs,
-                                             real_t (*H)[3][4], float (*xi2)[4]) {
+                                             BatchHermite<real_t>& bh) {
     constexpr int T = 8 * JW;
-    using vec_t = typename std::conditional<sizeof(real_t) == 8, double2, float4>::type;
-    constexpr int VE = 16 / sizeof(real_t), VPR = JW / VE;
     int const tid = threadIdx.x, j = slice * JW + jl;
-    if (a.add_local && b1 > b0) {
-        float const R2 = float(a.hgrid[3] * a.hgrid[3]);
-        for (uint32_t b = b0; b < b1; ++b) {
-            AddEntry const e = a.add_entry[b];
-            int const L = int(e.L);
-            if (L > 5) continue;  // done by k_sho_add_wide
-            int const nc = ((L + 1) * (L + 2) * (L + 3)) / 6;
-            __syncthreads();
-            stage_hermite<real_t>(H, xi2, a.htab, a.xtab, e.slot, L, tid, T);
-            {   // [coefficient][plane][JW]
-                real_t const* src = a.dcoef + (size_t(e.coef0) * a.nCols + col) * 128 + slice * JW;
-                for (int v = tid; v < 2 * nc * VPR; v += T) {
-                    int const row = v / VPR, cv = v % VPR;  // row = coefficient*2 + plane
-                    *reinterpret_cast<vec_t*>(cs + row * JW + cv * VE) =
-                        *reinterpret_cast<vec_t const*>(src + size_t(row >> 1) * a.nCols * 128 + (row & 1) * 64 + cv * VE);
-                }
+    if (a.add_local) {
+        int const zqu = __builtin_amdgcn_readfirstlane(zq);   // uniform within a wave
+        for (uint32_t b = b0; b < b1;) {
+            uint32_t const be = stage_batch<real_t, JW, T, 56>(a, b, b1, col, slice * JW, cs, bh);
+            real_t const* c = cs + p * JW + jl;
+            for (int q = 0; b < be; ++b) {
+                AddEntry const e = a.add_entry[b];
+                if (e.L > 5) continue;
+                uint32_t const in = uint32_t(a.smask[e.slot] >> (16 * zqu)) & 0xffff;
+                sho_add_regs<real_t, 0, 5>(acc, bh.H[q], in, c, 2 * JW, zq, int(e.L));
+                c += ((e.L + 1) * (e.L + 2) * (e.L + 3)) / 6 * (2 * JW);
+                ++q;
             }
-            __syncthreads();
-            sho_add_regs<real_t>(acc, H, xi2, R2, cs + p * JW + jl, 2 * JW, zq, L);
         }
     }
 
@@ -1021,8 +1053,7 @@ __global__ __launch_bounds__(8 * JW) void k_plane(LocalArgs<real_t> a) {
     constexpr int NSLICE = 64 / JW;
     __shared__ real_t xs[2 * 64 * JW];
     __shared__ __align__(16) real_t cs[2 * 56 * JW];   // add-back coefficients (numax <= 5), then the (x, y) sums
-    __shared__ real_t H[8][3][4];
-    __shared__ float xi2[3][4];
+    __shared__ BatchHermite<real_t> bh;
 
     uint64_t lin = blockIdx.x;
     if (a.per_xcd) lin = uint64_t(blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
@@ -1089,7 +1120,7 @@ __global__ __launch_bounds__(8 * JW) void k_plane(LocalArgs<real_t> a) {
     }
 
     plane_finish<real_t, JW>(a, blk, h.w[IH_COL], h.w[IH_ADD0], h.w[IH_ADD1], slice, p, zq, jl, acc, xsp, xso, cs,
-                             H, xi2);
+                             bh);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1177,12 +1208,13 @@ __device__ __forceinline__ void xline_layer(real_t (&t)[Lane<real_t>::n][L + 1],
 }
 
 // SHO add-back of one atom image (numax L) into the x-line (y, z) of a lane: the coefficients c[iz][iy][ix]
-// (ix fastest) are contracted with H_z(z) H_y(y) first, t[ix], then t with H_x at the 4 points of the line.
-// The z layers run in a rolled loop, so that one layer of coefficients at a time is loaded ahead.
+// (ix fastest) are contracted with H_z(z) H_y(y) first, t[ix], then t with H_x at the 4 points of the line; in: the
+// line's points inside the projection sphere (4 bits).  The z layers run in a rolled loop, so that one layer of
+// coefficients at a time is loaded ahead (unrolled, the kernel takes 256 VGPRs).
 // cs points to coefficient 0 of the lane's plane and first column; consecutive coefficients are cstride apart.
 template <typename real_t, int L>
-__device__ __forceinline__ void sho_xline(Lane<real_t> (&acc)[4], real_t const (*H)[3][4], float const (*xi2)[4],
-                                          float R2, real_t const* cs, int cstride, int y, int z) {
+__device__ __forceinline__ void sho_xline(Lane<real_t> (&acc)[4], real_t const (*H)[3][4], uint32_t in, real_t const* cs,
+                                          int cstride, int y, int z) {
     constexpr int CPL = Lane<real_t>::n;
     real_t t[CPL][L + 1];
 #pragma unroll
@@ -1204,13 +1236,13 @@ __device__ __forceinline__ void sho_xline(Lane<real_t> (&acc)[4], real_t const (
     }
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        bool const in = sho_inside(xi2, R2, z, y, q);
+        bool const inside = (in >> q) & 1;
 #pragma unroll
         for (int c = 0; c < CPL; ++c) {
             real_t v = 0;
 #pragma unroll
             for (int ix = 0; ix <= L; ++ix) v += t[c][ix] * H[ix][0][q];
-            acc[q].v[c] += in ? v : real_t(0);
+            acc[q].v[c] += inside ? v : real_t(0);
         }
     }
 }
@@ -1270,9 +1302,8 @@ void k_lines(LocalArgs<real_t> a) {
     constexpr int CPL = L16::n, LQ = JW / CPL, T = LQ * 32;
     constexpr int NSLICE = 64 / JW;
     __shared__ __align__(16) real_t xs[2 * 64 * JW];   // the slice [plane][point][column]
-    __shared__ __align__(16) real_t ya[2 * 64 * JW];   // y + z stencil sums; then the coefficients of an image
-    __shared__ real_t H[8][3][4];
-    __shared__ float xi2[3][4];
+    __shared__ __align__(16) real_t ya[2 * 64 * JW];   // y + z stencil sums; then the coefficients of a batch of images
+    __shared__ BatchHermite<real_t> bh;
 
     uint64_t lin = blockIdx.x;
     if (a.per_xcd) lin = uint64_t(blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
@@ -1366,34 +1397,25 @@ void k_lines(LocalArgs<real_t> a) {
     }
 
     // ---- SHO add-back of the atom images (numax <= 5) touching the block; coefficients staged in ya ----
-    uint32_t const b0 = h.w[IH_ADD0], b1 = h.w[IH_ADD1];
-    if (a.add_local && b1 > b0) {
-        uint32_t const col = h.w[IH_COL];
-        float const R2 = float(a.hgrid[3] * a.hgrid[3]);
-        constexpr int VPR = JW / CPL;
-        for (uint32_t b = b0; b < b1; ++b) {
-            AddEntry const e = a.add_entry[b];
-            int const L = int(e.L);
-            if (L > 5) continue;  // done by k_sho_add_wide
-            int const nc = ((L + 1) * (L + 2) * (L + 3)) / 6;
-            __syncthreads();   // ya (the stencil sums, or the previous image) is no longer read
-            stage_hermite<real_t>(H, xi2, a.htab, a.xtab, e.slot, L, tid, T);
-            {   // [coefficient][plane][JW]
-                real_t const* src = a.dcoef + (size_t(e.coef0) * a.nCols + col) * 128 + slice * JW;
-                for (int v = tid; v < 2 * nc * VPR; v += T) {
-                    int const row = v / VPR, cv = v % VPR;  // row = coefficient*2 + plane
-                    st16(ya + row * JW + cv * CPL, ld16(src + size_t(row >> 1) * a.nCols * 128 + (row & 1) * 64 + cv * CPL));
-                }
-            }
-            __syncthreads();
+    if (a.add_local) {
+        uint32_t const b1 = h.w[IH_ADD1];
+        for (uint32_t b = h.w[IH_ADD0]; b < b1;) {
+            uint32_t const be = stage_batch<real_t, JW, T, 64>(a, b, b1, h.w[IH_COL], slice * JW, ya, bh);
             real_t const* cs = ya + p * JW + jc;
-            switch (L) {
-                case 0: sho_xline<real_t, 0>(acc, H, xi2, R2, cs, 2 * JW, la, lb); break;
-                case 1: sho_xline<real_t, 1>(acc, H, xi2, R2, cs, 2 * JW, la, lb); break;
-                case 2: sho_xline<real_t, 2>(acc, H, xi2, R2, cs, 2 * JW, la, lb); break;
-                case 3: sho_xline<real_t, 3>(acc, H, xi2, R2, cs, 2 * JW, la, lb); break;
-                case 4: sho_xline<real_t, 4>(acc, H, xi2, R2, cs, 2 * JW, la, lb); break;
-                default: sho_xline<real_t, 5>(acc, H, xi2, R2, cs, 2 * JW, la, lb); break;
+            for (int q = 0; b < be; ++b) {
+                AddEntry const e = a.add_entry[b];
+                if (e.L > 5) continue;
+                uint32_t const in = uint32_t(a.smask[e.slot] >> ix0) & 15;
+                switch (e.L) {
+                    case 0: sho_xline<real_t, 0>(acc, bh.H[q], in, cs, 2 * JW, la, lb); break;
+                    case 1: sho_xline<real_t, 1>(acc, bh.H[q], in, cs, 2 * JW, la, lb); break;
+                    case 2: sho_xline<real_t, 2>(acc, bh.H[q], in, cs, 2 * JW, la, lb); break;
+                    case 3: sho_xline<real_t, 3>(acc, bh.H[q], in, cs, 2 * JW, la, lb); break;
+                    case 4: sho_xline<real_t, 4>(acc, bh.H[q], in, cs, 2 * JW, la, lb); break;
+                    default: sho_xline<real_t, 5>(acc, bh.H[q], in, cs, 2 * JW, la, lb); break;
+                }
+                cs += ((e.L + 1) * (e.L + 2) * (e.L + 3)) / 6 * (2 * JW);
+                ++q;
             }
         }
     }
@@ -1467,13 +1489,11 @@ __global__ __launch_bounds__(256) void k_sho_add_mfma(LocalArgs<real_t> a, uint3
     constexpr int NCP = 64;
     __shared__ real_t P[64 * NCP];   // [point][coefficient]
     __shared__ real_t H[6][3][4];
-    __shared__ float xi2[3][4];
     __shared__ uint16_t sxyz[NCP];   // coefficient s -> ix | iy << 4 | iz << 8 of the current image's numax
     uint32_t const blk = blocks[blockIdx.x];
     uint32_t const col = a.colindx[blk];
     if (col_active && !col_active[col]) return;
     int const tid = threadIdx.x, lane = tid & 63, w = tid >> 6, kl = lane >> 4;
-    float const R2 = float(a.hgrid[3] * a.hgrid[3]);
     acc_t acc[4][2];
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt)
@@ -1486,7 +1506,8 @@ __global__ __launch_bounds__(256) void k_sho_add_mfma(LocalArgs<real_t> a, uint3
         if (L > 5) continue;   // added by k_sho_add_wide
         int const nc = ((L + 1) * (L + 2) * (L + 3)) / 6;
         __syncthreads();   // P of the previous image is no longer read
-        stage_hermite<real_t>(H, xi2, a.htab, a.xtab, e.slot, L, tid, 256);
+        uint64_t const in = a.smask[e.slot];
+        stage_hermite<real_t>(H, a.htab, e.slot, L, tid, 256);
         if (tid == 0) {
             int q = 0;
             for (int iz = 0; iz <= L; ++iz)
@@ -1500,7 +1521,7 @@ __global__ __launch_bounds__(256) void k_sho_add_mfma(LocalArgs<real_t> a, uint3
             int const xx = i & 3, yy = (i >> 2) & 3, zz = i >> 4;
             uint16_t const code = sxyz[c];
             real_t v = 0;
-            if (code != 0xFFFF && sho_inside(xi2, R2, zz, yy, xx))
+            if (code != 0xFFFF && ((in >> i) & 1))
                 v = H[code & 15][0][xx] * H[(code >> 4) & 15][1][yy] * H[code >> 8][2][zz];
             P[e] = v;
         }
@@ -1534,30 +1555,56 @@ __global__ __launch_bounds__(256) void k_sho_add_mfma(LocalArgs<real_t> a, uint3
             }
 }
 
-// SHO add-back of the atom images with numax 6 or 7, y += P d, on the blocks listed in blocks[]: one work-group of
-// 512 threads = (column j, plane p, z plane zq) per block, taking the block's wide images one after the other, so
-// that no two work-groups update the same block.  Runs after the local kernel (which adds numax <= 5).
+// SHO add-back of the atom images with numax 6 or 7, y += P d, on the blocks listed in blocks[], after the local kernel
+// (which adds numax <= 5).  One work-group of 8 JS threads per (block, JS columns): thread (j, p, zq) holds the 16
+// points of z plane zq of one column and plane of y in registers, and the block's wide images are added one after the
+// other from LDS copies of their coefficients, so that no two work-groups update the same values and y is read and
+// written once.  JS fills 128-byte lines.
 template <typename real_t>
-__global__ __launch_bounds__(512) void k_sho_add_wide(LocalArgs<real_t> a, uint32_t const* __restrict__ blocks,
-                                                      uint8_t const* __restrict__ col_active) {
+__global__ __launch_bounds__(1024 / sizeof(real_t)) void k_sho_add_wide(LocalArgs<real_t> a,
+                                                                        uint32_t const* __restrict__ blocks,
+                                                                        uint8_t const* __restrict__ col_active) {
+    typedef real_t __attribute__((ext_vector_type(16 / sizeof(real_t)))) vec_t;
+    constexpr int JS = 128 / sizeof(real_t), T = 8 * JS, NS = 64 / JS, VE = 16 / sizeof(real_t), VPR = JS / VE;
+    constexpr int NCMAX = Sho<7>::n3;
+    constexpr int NV = (2 * NCMAX * VPR + T - 1) / T;   // 16-byte vectors of coefficients per thread
+    __shared__ __align__(16) real_t cs[2 * NCMAX * JS];   // [coefficient][plane][JS]
     __shared__ real_t H[8][3][4];
-    __shared__ float xi2[3][4];
-    uint32_t const blk = blocks[blockIdx.x];
+    uint32_t const blk = blocks[blockIdx.x / NS];
+    int const slice = blockIdx.x % NS;
     uint32_t const col = a.colindx[blk];
     if (col_active && !col_active[col]) return;
-    int const tid = threadIdx.x, j = tid & 63, p = (tid >> 6) & 1, zq = tid >> 7;
-    float const R2 = float(a.hgrid[3] * a.hgrid[3]);
-    real_t* yb = a.y + size_t(blk) * NBLK + p * 4096 + j;   // ys stride 64 for the direct update of y
+    int const tid = threadIdx.x, jl = tid % JS, p = (tid / JS) & 1, zq = tid / (2 * JS);
+    real_t* yb = a.y + size_t(blk) * NBLK + p * 4096 + zq * 1024 + slice * JS + jl;
+    real_t acc[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) acc[k] = yb[k * 64];
     for (uint32_t b = a.add_start[blk]; b < a.add_start[blk + 1]; ++b) {
         AddEntry const e = a.add_entry[b];
         int const L = int(e.L);
         if (L <= 5) continue;   // added by the local kernel
-        __syncthreads();        // H of the previous image is no longer read
-        stage_hermite<real_t>(H, xi2, a.htab, a.xtab, e.slot, L, tid, 512);
+        int const rows = ((L + 1) * (L + 2) * (L + 3)) / 3;
+        vec_t t[NV];
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+            int const v = k * T + tid, row = v / VPR, cv = v % VPR;   // row = coefficient * 2 + plane
+            if (row < rows)
+                t[k] = *reinterpret_cast<vec_t const*>(a.dcoef + (size_t(e.coef0 + (row >> 1)) * a.nCols + col) * 128 +
+                                                       (row & 1) * 64 + slice * JS + cv * VE);
+        }
+        __syncthreads();        // the previous image's coefficients are no longer read
+        stage_hermite<real_t>(H, a.htab, e.slot, L, tid, T);
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+            int const v = k * T + tid, row = v / VPR, cv = v % VPR;
+            if (row < rows) *reinterpret_cast<vec_t*>(cs + row * JS + cv * VE) = t[k];
+        }
         __syncthreads();
-        real_t const* dsrc = a.dcoef + (size_t(e.coef0) * a.nCols + col) * 128 + p * 64 + j;
-        sho_add_atom<real_t, 7>(yb, 64, H, xi2, R2, dsrc, size_t(a.nCols) * 128, zq, L);
+        uint32_t const in = uint32_t(a.smask[e.slot] >> (16 * zq)) & 0xffff;
+        sho_add_regs<real_t, 6, 7>(acc, H, in, cs + p * JS + jl, 2 * JS, zq, L);
     }
+#pragma unroll
+    for (int k = 0; k < 16; ++k) yb[k * 64] = acc[k];
 }
 
 template <typename T>
@@ -1817,9 +1864,9 @@ int device_upload_plan(Plan const& p, DevicePlan& d, std::string& err) {
             if ((s = dupload(d, dimg, simg, err))) return s;
             if ((s = dupload(d, drow, srow, err))) return s;
             if ((s = dalloc(d, d.htab, ns * 96, err))) return s;
-            if ((s = dalloc(d, d.xtab, ns * 12, err))) return s;
+            if ((s = dalloc(d, d.smask, ns, err))) return s;
             if (!d.slot_map.empty()) {
-                hipLaunchKernelGGL(k_hermite_table, dim3(uint32_t(d.slot_map.size())), dim3(64), 0, 0, d.htab, d.xtab,
+                hipLaunchKernelGGL(k_hermite_table, dim3(uint32_t(d.slot_map.size())), dim3(64), 0, 0, d.htab, d.smask,
                                    dimg, drow, d.image_pos, d.image_lmax, d.row_pos, p.hg[0], p.hg[1], p.hg[2], p.r_proj);
                 HIP_TRY(hipGetLastError());
                 HIP_TRY(hipDeviceSynchronize());
@@ -2030,9 +2077,9 @@ int device_action(DevicePlan& d, ActionScalars const& s, real_t* y, real_t const
             uint32_t const* bucket = d.bucket_chunks + d.bucket_start[L];
 #define LAUNCH_PRJ(LL) hipLaunchKernelGGL((k_sho_project<real_t, LL>), dim3(n), dim3(128), 0, stream, ws.partial, x, \
                 d.chunks, bucket, d.chunk_coef, d.prj_blocks, d.rowindx, d.row_pos, d.image_pos, \
-                s.hgrid[0], s.hgrid[1], s.hgrid[2], s.hgrid[3], d.col_active, d.htab, d.xtab, d.prj_slot)
+                s.hgrid[0], s.hgrid[1], s.hgrid[2], s.hgrid[3], d.col_active, d.htab, d.smask, d.prj_slot)
 #define LAUNCH_MFMA(LL) hipLaunchKernelGGL((k_sho_project_mfma<real_t, LL>), dim3(n), dim3(256), 0, stream, ws.partial, \
-                x, d.chunks, bucket, d.chunk_coef, d.prj_blocks, s.hgrid[3], d.col_active, d.htab, d.xtab, d.prj_slot)
+                x, d.chunks, bucket, d.chunk_coef, d.prj_blocks, d.col_active, d.htab, d.smask, d.prj_slot)
             if (d.prj_engine[sizeof(real_t) == 8 ? 0 : 1] == 1 && L <= 5) {   // the dense form on the matrix cores
                 switch (L) {
                     case 0: LAUNCH_MFMA(0); break; case 1: LAUNCH_MFMA(1); break;
@@ -2076,7 +2123,7 @@ int device_action(DevicePlan& d, ActionScalars const& s, real_t* y, real_t const
     a.add_entry = reinterpret_cast<AddEntry const*>(d.add_entry);
     a.nitems = d.active_order ? d.n_active : d.nnzb;
     a.E_col = d.E_col;
-    a.htab = d.htab; a.xtab = d.xtab;
+    a.htab = d.htab; a.smask = d.smask;
     a.dot = dot;
     int const engine = d.prj_engine[sizeof(real_t) == 8 ? 0 : 1];
     a.add_local = (engine == 1) ? 0 : 1;
@@ -2118,8 +2165,10 @@ int device_action(DevicePlan& d, ActionScalars const& s, real_t* y, real_t const
         HIP_TRY(hipGetLastError());
     }
     if (d.n_wide_blocks > 0) {
-        hipLaunchKernelGGL((k_sho_add_wide<real_t>), dim3(d.n_wide_blocks), dim3(512), 0, stream, a, d.wide_blocks,
-                           d.col_active);
+        uint64_t const wide = uint64_t(d.n_wide_blocks) * (64 * sizeof(real_t) / 128);   // column slices of 128 bytes
+        if (wide > 0x7fffffffull) { err = "too many blocks for one launch"; return 1; }
+        hipLaunchKernelGGL((k_sho_add_wide<real_t>), dim3(uint32_t(wide)), dim3(1024 / sizeof(real_t)), 0, stream, a,
+                           d.wide_blocks, d.col_active);
         HIP_TRY(hipGetLastError());
     }
     return 0;
@@ -2303,7 +2352,7 @@ static int project_collect(DevicePlan& d, ActionScalars const& s, double const* 
         uint32_t const* bucket = d.bucket_chunks + d.bucket_start[L];
 #define LAUNCH_PRJ(LL) hipLaunchKernelGGL((k_sho_project<double, LL>), dim3(n), dim3(128), 0, stream, ws.partial, vec, \
         d.chunks, bucket, d.chunk_coef, d.prj_blocks, d.rowindx, d.row_pos, d.image_pos, \
-        s.hgrid[0], s.hgrid[1], s.hgrid[2], s.hgrid[3], (uint8_t const*)nullptr, d.htab, d.xtab, d.prj_slot)
+        s.hgrid[0], s.hgrid[1], s.hgrid[2], s.hgrid[3], (uint8_t const*)nullptr, d.htab, d.smask, d.prj_slot)
         switch (L) {
             case 0: LAUNCH_PRJ(0); break; case 1: LAUNCH_PRJ(1); break;
             case 2: LAUNCH_PRJ(2); break; case 3: LAUNCH_PRJ(3); break;

@@ -69,9 +69,10 @@ struct DevicePlan {
     uint32_t* items = nullptr;         // [nnzb][head_words] in processing order
     int head_words = 16;
     uint32_t* add_entry = nullptr;     // [add nnz][4]: image, numax, Hermite slot, first coefficient of the image
-    // Hermite functions per (atom image, target row) slot: htab[slot][8][3][4], xtab[slot][3][4] = xi^2
+    // Hermite functions per (atom image, target row) slot: htab[slot][8][3][4], and the points inside the projection
+    // sphere, smask[slot]
     double* htab = nullptr;
-    float* xtab = nullptr;
+    uint64_t* smask = nullptr;
     uint32_t* prj_slot = nullptr;      // [projection blocks] slot of each chunk block
     uint32_t nslots = 0;
     std::map<uint64_t, uint32_t> slot_map;  // (image << 32 | row) -> slot, during upload only
