@@ -511,9 +511,10 @@ struct LocalArgs {
 // Contracted z first (one value H_z[iz](zq) per thread), then y and x row by row: (L+1)(L+2)(L+3)/6 +
 // 4 (L+1)(L+2)/2 + 16 (L+1) FMAs.  All loops are unrolled, with a scheduling barrier after every z layer so that at
 // most one layer of coefficients is loaded ahead (rolled layers with a run-time size cost a copy of all sums per
-// layer: more moves than FMAs); ROLL keeps the row loop rolled (out must then accept a run-time row y).
+// layer: more moves than FMAs); ROLL keeps the row loop rolled (out must then accept a run-time row y).  TIGHT adds a
+// barrier after every row, for callers that are held to fewer registers.
 // dsrc points to coefficient 0 of this thread's (plane, column); consecutive coefficients are dstride apart.
-template <typename real_t, int L, bool ROLL, typename Out>
+template <typename real_t, int L, bool ROLL, bool TIGHT, typename Out>
 __device__ __forceinline__ void sho_plane(real_t const (*H)[3][4], real_t const* __restrict__ dsrc, size_t dstride,
                                           int zq, Out&& out) {
     constexpr int n2 = ((L + 1) * (L + 2)) / 2;
@@ -548,6 +549,7 @@ __device__ __forceinline__ void sho_plane(real_t const (*H)[3][4], real_t const*
             for (int ix = 0; ix <= L; ++ix) v += by[ix] * H[ix][0][xx];
             out(y, xx, v);
         }
+        if constexpr (TIGHT) __builtin_amdgcn_sched_barrier(0);
     };
     if constexpr (ROLL) {
 #pragma unroll 1
@@ -559,14 +561,14 @@ __device__ __forceinline__ void sho_plane(real_t const (*H)[3][4], real_t const*
 }
 
 // sho_plane for a run-time numax LMIN <= L <= LMAX
-template <typename real_t, int LMIN, int LMAX, bool ROLL, typename Out>
+template <typename real_t, int LMIN, int LMAX, bool ROLL, bool TIGHT, typename Out>
 __device__ __forceinline__ void sho_plane_any(real_t const (*H)[3][4], real_t const* __restrict__ dsrc, size_t dstride,
                                               int zq, int L, Out&& out) {
     if constexpr (LMIN < LMAX) {
-        if (L == LMIN) sho_plane<real_t, LMIN, ROLL>(H, dsrc, dstride, zq, out);
-        else sho_plane_any<real_t, LMIN + 1, LMAX, ROLL>(H, dsrc, dstride, zq, L, out);
+        if (L == LMIN) sho_plane<real_t, LMIN, ROLL, TIGHT>(H, dsrc, dstride, zq, out);
+        else sho_plane_any<real_t, LMIN + 1, LMAX, ROLL, TIGHT>(H, dsrc, dstride, zq, L, out);
     } else {
-        sho_plane<real_t, LMAX, ROLL>(H, dsrc, dstride, zq, out);
+        sho_plane<real_t, LMAX, ROLL, TIGHT>(H, dsrc, dstride, zq, out);
     }
 }
 
@@ -575,7 +577,7 @@ __device__ __forceinline__ void sho_plane_any(real_t const (*H)[3][4], real_t co
 template <typename real_t>
 __device__ __forceinline__ void sho_add_atom(real_t* __restrict__ ys, int ostride, real_t const (*H)[3][4], uint64_t in,
                                              real_t const* __restrict__ dsrc, size_t dstride, int zq, int L) {
-    sho_plane_any<real_t, 0, 5, true>(H, dsrc, dstride, zq, L, [&](int y, int xx, real_t v) {
+    sho_plane_any<real_t, 0, 5, true, false>(H, dsrc, dstride, zq, L, [&](int y, int xx, real_t v) {
         real_t& o = ys[(zq * 16 + y * 4 + xx) * ostride];
         o += ((in >> (zq * 16 + y * 4 + xx)) & 1) ? v : real_t(0);
     });
@@ -583,10 +585,10 @@ __device__ __forceinline__ void sho_add_atom(real_t* __restrict__ ys, int ostrid
 
 // SHO add-back of one atom image (LMIN <= numax <= LMAX) into 16 register accumulators (z plane zq of one column and
 // plane); in: the plane's points inside the projection sphere (16 bits)
-template <typename real_t, int LMIN, int LMAX>
+template <typename real_t, int LMIN, int LMAX, bool TIGHT = false>
 __device__ __forceinline__ void sho_add_regs(real_t (&out)[16], real_t const (*H)[3][4], uint32_t in,
                                              real_t const* __restrict__ dsrc, size_t dstride, int zq, int L) {
-    sho_plane_any<real_t, LMIN, LMAX, false>(H, dsrc, dstride, zq, L, [&](int y, int xx, real_t v) {
+    sho_plane_any<real_t, LMIN, LMAX, false, TIGHT>(H, dsrc, dstride, zq, L, [&](int y, int xx, real_t v) {
         out[y * 4 + xx] += ((in >> (y * 4 + xx)) & 1) ? v : real_t(0);
     });
 }
@@ -656,6 +658,27 @@ __device__ __forceinline__ uint32_t stage_batch(LocalArgs<real_t> const& a, uint
     }
     __syncthreads();
     return b;
+}
+
+// the atom images (numax <= 5) of add-list entries b0 .. b1 - 1, added to out: the z plane zq of this thread's column,
+// which is column c0 + jl of plane p.  cs: LDS for CAP coefficients [coefficient][plane][JW].
+// Contains barriers: every thread of the work-group calls it; after it cs may still be read by other threads.
+template <typename real_t, int JW, int T, int CAP, bool TIGHT = false>
+__device__ __forceinline__ void add_images(LocalArgs<real_t> const& a, uint32_t b0, uint32_t b1, uint32_t col, int c0,
+                                           int p, int jl, int zq, real_t* cs, BatchHermite<real_t>& bh,
+                                           real_t (&out)[16]) {
+    for (uint32_t b = b0; b < b1;) {
+        uint32_t const be = stage_batch<real_t, JW, T, CAP>(a, b, b1, col, c0, cs, bh);
+        real_t const* c = cs + p * JW + jl;
+        for (int q = 0; b < be; ++b) {
+            AddEntry const e = a.add_entry[b];
+            if (e.L > 5) continue;
+            uint32_t const in = uint32_t(a.smask[e.slot] >> (16 * zq));
+            sho_add_regs<real_t, 0, 5, TIGHT>(out, bh.H[q], in, c, 2 * JW, zq, int(e.L));
+            c += ((e.L + 1) * (e.L + 2) * (e.L + 3)) / 6 * (2 * JW);
+            ++q;
+        }
+    }
 }
 
 // value of a neighbour block at point e (a compile-time element offset from the uniform pointer b) and byte
@@ -996,21 +1019,8 @@ __device__ __forceinline__ void plane_finish(LocalArgs<real_t> const& a, uint64_
                                              BatchHermite<real_t>& bh) {
     constexpr int T = 8 * JW;
     int const tid = threadIdx.x, j = slice * JW + jl;
-    if (a.add_local) {
-        int const zqu = __builtin_amdgcn_readfirstlane(zq);   // uniform within a wave
-        for (uint32_t b = b0; b < b1;) {
-            uint32_t const be = stage_batch<real_t, JW, T, 56>(a, b, b1, col, slice * JW, cs, bh);
-            real_t const* c = cs + p * JW + jl;
-            for (int q = 0; b < be; ++b) {
-                AddEntry const e = a.add_entry[b];
-                if (e.L > 5) continue;
-                uint32_t const in = uint32_t(a.smask[e.slot] >> (16 * zqu)) & 0xffff;
-                sho_add_regs<real_t, 0, 5>(acc, bh.H[q], in, c, 2 * JW, zq, int(e.L));
-                c += ((e.L + 1) * (e.L + 2) * (e.L + 3)) / 6 * (2 * JW);
-                ++q;
-            }
-        }
-    }
+    if (a.add_local)   // zq is uniform within a wave
+        add_images<real_t, JW, T, 56>(a, b0, b1, col, slice * JW, p, jl, __builtin_amdgcn_readfirstlane(zq), cs, bh, acc);
 
     real_t* dst = a.y + blk * NBLK + size_t(p * 4096 + j) + size_t(zq * 16) * 64;
 #pragma unroll
@@ -1289,16 +1299,22 @@ __device__ __forceinline__ void phase_lines(LocalArgs<real_t> const& a, int d, I
 
 // PF: directions whose neighbour lines are issued before the first barrier (3: all; 2: x and y, z after the x
 // stencil; 1: x, then y after the x stencil and z after the y stencil) -- loads in flight against occupancy.
-// The FP64 shape with 16 columns and PF 2 is held to 128 VGPRs (4 waves per SIMD); with image phases the shuffles push
+// The 8th-order shapes without images and with PF 2 (in FP64 that of 16 columns) are held to 128 VGPRs (4 waves per
+// SIMD; FP32, 158k blocks: 3,347 us against 3,616 with 154 VGPRs and 3 waves); with image phases the shuffles push
 // every 8th-order shape past 168, so those are held to 168 (3 waves, 5 spills; at 128 they spill 53).  Measured, FP64,
 // 16 columns, 2 directions: 512 blocks at a k-point 49 -> 32 us, 1,024 blocks 87 -> 57, 6,144 blocks 705 -> 368 against
 // loading the other plane's lines as well; 45,896 blocks without images 2,118 -> 2,050 us from loading the potential
 // before the barrier.  16th order: unbounded (184 VGPRs; held to 168, 11,474 blocks FP64 take 941 us instead of 829).
 template <typename real_t, int NH, bool IMG, int JW, int PF>
+constexpr bool lines_four_waves() {
+    return NH == 1 && !IMG && PF == 2 && (sizeof(real_t) == 4 || JW == 16);
+}
+template <typename real_t, int NH, bool IMG, int JW, int PF>
 __global__ __launch_bounds__((JW / Lane<real_t>::n) * 32,
-                             (sizeof(real_t) == 8 && JW == 16 && PF == 2 && !IMG) ? 4 : (IMG && NH == 1) ? 3 : 1)
+                             (lines_four_waves<real_t, NH, IMG, JW, PF>() ? 4 : (IMG && NH == 1) ? 3 : 1))
 void k_lines(LocalArgs<real_t> a) {
     using L16 = Lane<real_t>;
+    constexpr bool W4 = lines_four_waves<real_t, NH, IMG, JW, PF>();
     constexpr int CPL = L16::n, LQ = JW / CPL, T = LQ * 32;
     constexpr int NSLICE = 64 / JW;
     __shared__ __align__(16) real_t xs[2 * 64 * JW];   // the slice [plane][point][column]
@@ -1397,25 +1413,47 @@ void k_lines(LocalArgs<real_t> a) {
     }
 
     // ---- SHO add-back of the atom images (numax <= 5) touching the block; coefficients staged in ya ----
-    if (a.add_local) {
-        uint32_t const b1 = h.w[IH_ADD1];
-        for (uint32_t b = h.w[IH_ADD0]; b < b1;) {
-            uint32_t const be = stage_batch<real_t, JW, T, 64>(a, b, b1, h.w[IH_COL], slice * JW, ya, bh);
-            real_t const* cs = ya + p * JW + jc;
-            for (int q = 0; b < be; ++b) {
-                AddEntry const e = a.add_entry[b];
-                if (e.L > 5) continue;
-                uint32_t const in = uint32_t(a.smask[e.slot] >> ix0) & 15;
-                switch (e.L) {
-                    case 0: sho_xline<real_t, 0>(acc, bh.H[q], in, cs, 2 * JW, la, lb); break;
-                    case 1: sho_xline<real_t, 1>(acc, bh.H[q], in, cs, 2 * JW, la, lb); break;
-                    case 2: sho_xline<real_t, 2>(acc, bh.H[q], in, cs, 2 * JW, la, lb); break;
-                    case 3: sho_xline<real_t, 3>(acc, bh.H[q], in, cs, 2 * JW, la, lb); break;
-                    case 4: sho_xline<real_t, 4>(acc, bh.H[q], in, cs, 2 * JW, la, lb); break;
-                    default: sho_xline<real_t, 5>(acc, bh.H[q], in, cs, 2 * JW, la, lb); break;
+    if (a.add_local && h.w[IH_ADD1] > h.w[IH_ADD0]) {
+        uint32_t const b1 = h.w[IH_ADD1], col = h.w[IH_COL];
+        if constexpr (sizeof(real_t) == 4) {
+            // FP32: for the add-back a thread takes a z plane of ONE column, as in k_plane, and the sums meet the x-lines
+            // in ya.  Contracted for a whole plane an image costs 236 FMAs per 16 points at numax 5, for x-lines of
+            // several columns 400 (158k blocks: 3,843 -> 3,347 us; without any add-back 2,893).  In FP64 the plane
+            // of a column needs 202 VGPRs, or spills at 128.
+            int const jl = tid % JW, pp = (tid / JW) & 1, zq = tid / (2 * JW);
+            real_t out[16];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) out[k] = 0;
+            add_images<real_t, JW, T, 64, W4>(a, h.w[IH_ADD0], b1, col, slice * JW, pp, jl, zq, ya, bh, out);
+            __syncthreads();   // the coefficients are no longer read
+#pragma unroll
+            for (int k = 0; k < 16; ++k) ya[(pp * 64 + zq * 16 + k) * JW + jl] = out[k];
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                L16 const s = ld16(ya + (p * 64 + ix0 + q) * JW + jc);
+#pragma unroll
+                for (int c = 0; c < CPL; ++c) acc[q].v[c] += s.v[c];
+            }
+        } else {
+            for (uint32_t b = h.w[IH_ADD0]; b < b1;) {
+                uint32_t const be = stage_batch<real_t, JW, T, 64>(a, b, b1, col, slice * JW, ya, bh);
+                real_t const* cs = ya + p * JW + jc;
+                for (int q = 0; b < be; ++b) {
+                    AddEntry const e = a.add_entry[b];
+                    if (e.L > 5) continue;
+                    uint32_t const in = uint32_t(a.smask[e.slot] >> ix0) & 15;
+                    switch (e.L) {
+                        case 0: sho_xline<real_t, 0>(acc, bh.H[q], in, cs, 2 * JW, la, lb); break;
+                        case 1: sho_xline<real_t, 1>(acc, bh.H[q], in, cs, 2 * JW, la, lb); break;
+                        case 2: sho_xline<real_t, 2>(acc, bh.H[q], in, cs, 2 * JW, la, lb); break;
+                        case 3: sho_xline<real_t, 3>(acc, bh.H[q], in, cs, 2 * JW, la, lb); break;
+                        case 4: sho_xline<real_t, 4>(acc, bh.H[q], in, cs, 2 * JW, la, lb); break;
+                        default: sho_xline<real_t, 5>(acc, bh.H[q], in, cs, 2 * JW, la, lb); break;
+                    }
+                    cs += ((e.L + 1) * (e.L + 2) * (e.L + 3)) / 6 * (2 * JW);
+                    ++q;
                 }
-                cs += ((e.L + 1) * (e.L + 2) * (e.L + 3)) / 6 * (2 * JW);
-                ++q;
             }
         }
     }
@@ -1600,7 +1638,7 @@ __global__ __launch_bounds__(1024 / sizeof(real_t)) void k_sho_add_wide(LocalArg
             if (row < rows) *reinterpret_cast<vec_t*>(cs + row * JS + cv * VE) = t[k];
         }
         __syncthreads();
-        uint32_t const in = uint32_t(a.smask[e.slot] >> (16 * zq)) & 0xffff;
+        uint32_t const in = uint32_t(a.smask[e.slot] >> (16 * zq));
         sho_add_regs<real_t, 6, 7>(acc, H, in, cs + p * JS + jl, 2 * JS, zq, L);
     }
 #pragma unroll
@@ -2015,7 +2053,11 @@ __global__ __launch_bounds__(64) void k_grad_atoms(double* __restrict__ gmat, do
 }
 
 // Local-kernel tile shapes.  kind 0: k_local (LDS accumulator), JW columns per work-group (16 or 32), LB
-// kinetic lines per thread in flight (1, 2, 4).  kind 1: k_plane (register accumulator), JW = 32 or 64.
+// kinetic lines per thread in flight (1, 2, 4).  kind 1: k_plane (register accumulator), JW = 32 or 64; its FP32
+// 8th-order shape of 32 columns, the default, is run by k_lines with 2 directions ahead, which adds the images in
+// the same plane form but reads and writes 16 bytes per lane: 158,112 blocks 3,347 us against 3,779 for k_plane,
+// 19,764 blocks 424 against 472, 1,461 blocks 31.1 against 35.2, 6,144 blocks with images 138 against 156, 64 blocks
+// 15.0 against 16.6.
 // kind 2: k_lines (16-byte lanes, line ownership), JW = 16 or 32, or 64 in FP32; LB = directions of neighbour
 // lines issued up front (3 or 2; 16th-order stencils issue one direction at a time).
 template <typename real_t, int NH, bool IMG>
@@ -2038,7 +2080,9 @@ static void launch_local(int kind, int jw, int lb, dim3 g, hipStream_t stream, L
             else KN(32, 3);
         }
     } else if (kind == 1) {
-        if (jw == 64) KP(64); else KP(32);
+        if (jw == 64) KP(64);
+        else if constexpr (sizeof(real_t) == 4 && NH == 1) KN(32, 2);   // the faster kernel on every plan measured
+        else KP(32);
     } else if (jw == 16) {
         if (lb == 1) KL(16, 1); else if (lb == 4) KL(16, 4); else KL(16, 2);
     } else {

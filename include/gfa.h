@@ -170,7 +170,8 @@ int gfa_action_part(gfa_plan* plan, int fp_bits, int part, void* y, const void* 
  *      No counterpart in the reference, whose kernels have fixed launch shapes. ---- */
 int gfa_autotune(gfa_plan* plan, int fp_bits, void* y, const void* x, void* stream, int reps, double* best_ms);
 /* pins the tile shape instead: kind 0 (LDS accumulator): columns per work-group 16 or 32, kinetic lines per
- * thread in flight 1, 2 or 4; kind 1 (register accumulator per z plane): columns 32 or 64, lines ignored;
+ * thread in flight 1, 2 or 4; kind 1 (register accumulator per z plane): columns 32 or 64, lines ignored
+ * (in FP32, for stencils up to the 8th order, 32 columns run as kind 2 with 2 lines, which is faster);
  * kind 2 (16-byte lanes, each thread owning one x-, y- and z-line): columns 16 or 32 (or 64 in FP32), lines = the
  * directions whose neighbour lines are loaded before the first stencil, 2 or 3 */
 int gfa_set_tile_shape(gfa_plan* plan, int fp_bits, int kind, int columns, int lines);
