@@ -1420,7 +1420,8 @@ void k_lines(LocalArgs<real_t> a) {
             // in ya.  Contracted for a whole plane an image costs 236 FMAs per 16 points at numax 5, for x-lines of
             // several columns 400 (158k blocks: 3,843 -> 3,347 us; without any add-back 2,893).  In FP64 the plane
             // of a column needs 202 VGPRs, or spills at 128.
-            int const jl = tid % JW, pp = (tid / JW) & 1, zq = tid / (2 * JW);
+            int const jl = tid % JW, pp = (tid / JW) & 1, zt = tid / (2 * JW);
+            int const zq = JW >= 32 ? __builtin_amdgcn_readfirstlane(zt) : zt;   // uniform within a wave from 32 columns
             real_t out[16];
 #pragma unroll
             for (int k = 0; k < 16; ++k) out[k] = 0;
@@ -1468,48 +1469,42 @@ void k_lines(LocalArgs<real_t> a) {
         // (x, y) = sum_i x_i y_i per column: plane 0 holds x_r, y_r (+ x_i), plane 1 x_i, y_i (+ x_r):
         // Re = sum x_r y_r - sum x_i y_i, Im = sum x_i y_r + sum x_r y_i; 4 products in the vector precision,
         // then FP64 over the 32 lines and planes of the work-group in a fixed order
-        real_t re_t[CPL], im_t[CPL];   // x of both planes at the x-line from the LDS copy of the slice
+        L16 re_v, im_v;   // x of both planes at the x-line from the LDS copy of the slice
 #pragma unroll
-        for (int c = 0; c < CPL; ++c) re_t[c] = im_t[c] = 0;
+        for (int c = 0; c < CPL; ++c) re_v.v[c] = im_v.v[c] = 0;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             L16 const xp = ld16(xs + (p * 64 + ix0 + q) * JW + jc), xo = ld16(xs + ((1 - p) * 64 + ix0 + q) * JW + jc);
 #pragma unroll
             for (int c = 0; c < CPL; ++c) {
-                re_t[c] += xp.v[c] * acc[q].v[c];
-                im_t[c] += xo.v[c] * acc[q].v[c];
+                re_v.v[c] += xp.v[c] * acc[q].v[c];
+                im_v.v[c] += xo.v[c] * acc[q].v[c];
             }
         }
-        // the lanes of one column group within a wave (lane bits LQ and up: plane and line) are summed with
-        // shuffles, then the waves' partial sums in LDS ([wave][re, im][JW], fits xs) in wave order
-        constexpr int NWAVE = T / 64;
-        double re[CPL], im[CPL];
 #pragma unroll
-        for (int c = 0; c < CPL; ++c) {
-            re[c] = (p == 1) ? -double(re_t[c]) : double(re_t[c]);
-            im[c] = double(im_t[c]);
-#pragma unroll
-            for (int o = LQ; o < 64; o <<= 1) {
-                re[c] += __shfl_xor(re[c], o, 64);
-                im[c] += __shfl_xor(im[c], o, 64);
-            }
-        }
-        __syncthreads();   // xs is free
-        double* red = reinterpret_cast<double*>(xs);
-        int const wave = tid >> 6, lane = tid & 63;
-        if (lane < LQ) {
-#pragma unroll
-            for (int c = 0; c < CPL; ++c) {
-                red[(wave * 2 + 0) * JW + jc + c] = re[c];
-                red[(wave * 2 + 1) * JW + jc + c] = im[c];
-            }
-        }
+        for (int c = 0; c < CPL; ++c) re_v.v[c] = (p == 1) ? -re_v.v[c] : re_v.v[c];
+        // through LDS, as re and im of [line and plane][column]: thread (column, re or im, part) sums 1 / PARTS of the
+        // 32 lines and planes in FP64, then the first 2 JW threads the parts; as shuffles within a wave this
+        // took 48 of 64 bits per thread in FP32 (inside a solve, 6,144 blocks with images 94.9 -> 86.3 us, 19,764 blocks
+        // without 310 -> 294; FP64, 1,024 blocks with images 50.2 -> 49.0)
+        constexpr int PARTS = T / (2 * JW), PER = 32 / PARTS;
+        __syncthreads();   // xs and ya are free
+        real_t* red = ya + (l * 2 + p) * (2 * JW) + jc;
+        st16(red, re_v);
+        st16(red + JW, im_v);
         __syncthreads();
-        if (tid < JW) {
-            double sr = 0, si = 0;
-            for (int w = 0; w < NWAVE; ++w) { sr += red[(w * 2 + 0) * JW + tid]; si += red[(w * 2 + 1) * JW + tid]; }
-            a.dot[(blk * 2 + 0) * 64 + slice * JW + tid] = sr;
-            a.dot[(blk * 2 + 1) * 64 + slice * JW + tid] = si;
+        int const cc = tid % (2 * JW), part = tid / (2 * JW);   // cc < JW: re, otherwise im
+        double sum = 0;
+#pragma unroll
+        for (int k = 0; k < PER; ++k) sum += double(ya[(part * PER + k) * (2 * JW) + cc]);
+        double* const tot = reinterpret_cast<double*>(xs);   // [part][re, im][JW]
+        tot[part * (2 * JW) + cc] = sum;
+        __syncthreads();
+        if (tid < 2 * JW) {
+            sum = 0;
+#pragma unroll
+            for (int k = 0; k < PARTS; ++k) sum += tot[k * (2 * JW) + tid];
+            a.dot[(blk * 2 + tid / JW) * 64 + slice * JW + tid % JW] = sum;
         }
     }
 }
