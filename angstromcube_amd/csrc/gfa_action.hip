@@ -25,6 +25,7 @@
 #include <mutex>
 #include <cmath>
 #include <cstdio>
+#include <cstring>
 #include <type_traits>
 
 namespace gfa {
@@ -1985,15 +1986,19 @@ __global__ __launch_bounds__(256) void k_grad_v_blocks(double* __restrict__ gpar
     }
 }
 
-// per cell block: the sum over the blocks that read its potential, in ascending block order
-__global__ __launch_bounds__(64) void k_grad_v_cells(double* __restrict__ gcell, double const* __restrict__ gpart,
+// per cell block (bx, by, bz): the sum over the blocks that read its potential, in ascending block order, written in
+// the caller's grid order [4 nbz][4 nby][4 nbx], so that the host copies it once and sorts nothing (a gradient on 64^3
+// points, 11,688 blocks, 903 -> 691 us with the entries of k_grad_atoms below spread over more waves)
+__global__ __launch_bounds__(64) void k_grad_v_cells(double* __restrict__ grid, double const* __restrict__ gpart,
                                                      uint32_t const* __restrict__ cell_start,
-                                                     uint32_t const* __restrict__ cell_blocks) {
-    uint32_t const v = blockIdx.x;
+                                                     uint32_t const* __restrict__ cell_blocks, uint32_t nbx,
+                                                     uint32_t nby) {
+    uint32_t const v = blockIdx.x, bx = v % nbx, by = (v / nbx) % nby, bz = v / nbx / nby;
     int const i = threadIdx.x;
     double acc = 0;
     for (uint32_t k = cell_start[v]; k < cell_start[v + 1]; ++k) acc += gpart[uint64_t(cell_blocks[k]) * 64 + i];
-    gcell[uint64_t(v) * 64 + i] = acc;
+    grid[((uint64_t(bz) * 4 + (i >> 4)) * (4 * uint64_t(nby)) + by * 4 + ((i >> 2) & 3)) * (4 * uint64_t(nbx)) + bx * 4 +
+         (i & 3)] = acc;
 }
 
 // atom coefficients of one vector: per (atom, column group) the image partials collected with the Bloch phase,
@@ -2014,36 +2019,124 @@ __global__ __launch_bounds__(256) void k_sho_collect(
     dst[64] = ai;
 }
 
-// per (atom a, row k): for every l, z_c = sum_j conj(cL[k][c][j]) cX[l][c][j];
-// gmat[a] = [-Im sum_c w_c z_c][k][l] (dL/dM entries times 1) and [-Im sum_c w_c (-E_c) z_c][k][l]
-__global__ __launch_bounds__(64) void k_grad_atoms(double* __restrict__ gmat, double const* __restrict__ cX,
-                                                   double const* __restrict__ cL, int8_t const* __restrict__ atom_lmax,
-                                                   uint32_t const* __restrict__ atom_starts,
-                                                   uint64_t const* __restrict__ atom_mat_off,
-                                                   double const* __restrict__ wE, uint32_t nCols) {
+// per (atom a, row k, entry l): z_c = sum_j conj(cL[k][c][j]) cX[l][c][j];
+// gmat[a] = [-Im sum_c w_c z_c][k][l] (dL/dM entries times 1) and [-Im sum_c w_c (-E_c) z_c][k][l].
+// A wave per entry, 4 per work-group: latency-bound (16 atoms, numax 3, 8 column groups: 6,400 waves; with a wave per row
+// looping over l, 320 waves, it took 70 us, now 11).
+__global__ __launch_bounds__(256) void k_grad_atoms(double* __restrict__ gmat, double const* __restrict__ cX,
+                                                    double const* __restrict__ cL, int8_t const* __restrict__ atom_lmax,
+                                                    uint32_t const* __restrict__ atom_starts,
+                                                    uint64_t const* __restrict__ atom_mat_off,
+                                                    double const* __restrict__ wE, uint32_t nCols) {
     uint32_t const a = blockIdx.x;
-    int const k = blockIdx.y, j = threadIdx.x;
+    int const k = blockIdx.y, l = blockIdx.z * 4 + (threadIdx.x >> 6), j = threadIdx.x & 63;
     int const L = atom_lmax[a];
     int const nc = ((L + 1) * (L + 2) * (L + 3)) / 6;
-    if (k >= nc) return;
+    if (k >= nc || l >= nc) return;   // uniform over the wave; no barrier below
     size_t const base = size_t(atom_starts[a]) * nCols * 128;
-    for (int l = 0; l < nc; ++l) {
-        double hr = 0, sr = 0;   // -Im of the two weighted sums
-        for (uint32_t c = 0; c < nCols; ++c) {
-            double const* pl = cL + base + (size_t(k) * nCols + c) * 128 + j;
-            double const* px = cX + base + (size_t(l) * nCols + c) * 128 + j;
-            double const lr = pl[0], li = pl[64], xr = px[0], xi = px[64];
-            double const zr = lr * xr + li * xi, zi = lr * xi - li * xr;   // conj(l) x
-            double const w_r = wE[4 * c], w_i = wE[4 * c + 1], v_r = wE[4 * c + 2], v_i = wE[4 * c + 3];
-            hr -= w_r * zi + w_i * zr;
-            sr -= v_r * zi + v_i * zr;
+    double const* pl = cL + base + size_t(k) * nCols * 128 + j;
+    double const* px = cX + base + size_t(l) * nCols * 128 + j;
+    double hr = 0, sr = 0;   // -Im of the two weighted sums
+#pragma unroll 2
+    for (uint32_t c = 0; c < nCols; ++c) {
+        double const lr = pl[size_t(c) * 128], li = pl[size_t(c) * 128 + 64];
+        double const xr = px[size_t(c) * 128], xi = px[size_t(c) * 128 + 64];
+        double const zr = lr * xr + li * xi, zi = lr * xi - li * xr;   // conj(l) x
+        double const w_r = wE[4 * c], w_i = wE[4 * c + 1], v_r = wE[4 * c + 2], v_i = wE[4 * c + 3];
+        hr -= w_r * zi + w_i * zr;
+        sr -= v_r * zi + v_i * zr;
+    }
+    hr = wave_sum(hr);
+    sr = wave_sum(sr);
+    if (j == 0) {
+        gmat[atom_mat_off[a] + size_t(k) * nc + l] = hr;
+        gmat[atom_mat_off[a] + size_t(nc) * nc + size_t(k) * nc + l] = sr;
+    }
+}
+
+// Atomic density matrices, the right projection of the collected coefficients c of X onto the same image
+// (SHOprj_right, include/green_dyadic.hxx:925-1036): D[i][j] = factor Im(phase sum_c sum_s c[i][c][s] p_j(c, s)) over the
+// 64 points s of every source block c.  One work-group per (image, row i); wave w takes the source blocks w, w + 4, ...
+// and a lane the entry j (nc <= 120: at most two), contracting x, y, z in turn (84 FMAs per component and block).
+// desc[image] = {first coefficient row of its atom, offset of its matrix (low, high word)}, the float bits of col_pos
+// follow.  As loops on the host, after a copy of all coefficients, this took about 150 us for 4 atoms of
+// numax 3 and 8 source blocks; here 8 us.
+__global__ __launch_bounds__(256) void k_density(double* __restrict__ D, double const* __restrict__ cX,
+                                                 double const* __restrict__ image_pos,
+                                                 int8_t const* __restrict__ image_lmax,
+                                                 double const* __restrict__ image_phase,
+                                                 uint32_t const* __restrict__ desc, uint32_t nai, uint32_t nCols,
+                                                 double hx, double hy, double hz, double rproj, double factor) {
+    __shared__ double A[4][2][64];      // masked coefficients of the wave's source block
+    __shared__ double H[4][8][3][4];
+    __shared__ float x2[4][3][4];
+    __shared__ double part[4][2][128];
+    uint32_t const img = blockIdx.x;
+    int const i = blockIdx.y, tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+    int const L = image_lmax[img], nc = ((L + 1) * (L + 2) * (L + 3)) / 6;
+    if (i >= nc) return;   // uniform over the work-group
+    float const* col_pos = reinterpret_cast<float const*>(desc + size_t(nai) * 3);
+    double const* src0 = cX + (size_t(desc[3 * size_t(img)]) + i) * nCols * 128 + lane;
+    int jx[2], jy[2], jz[2];   // exponents of the lane's entries
+    for (int q = 0; q < 2; ++q) {
+        int r = lane + 64 * q, iz = 0, iy = 0;
+        if (r >= nc) r = 0;
+        while (r >= ((L - iz + 1) * (L - iz + 2)) / 2) { r -= ((L - iz + 1) * (L - iz + 2)) / 2; ++iz; }
+        while (r >= L - iz - iy + 1) { r -= L - iz - iy + 1; ++iy; }
+        jx[q] = r; jy[q] = iy; jz[q] = iz;
+    }
+    int const nq = nc > 64 ? 2 : 1;
+    double sre[2] = {0, 0}, sim[2] = {0, 0};
+    float const R2 = float(rproj * rproj);
+    double const hgrid[4] = {hx, hy, hz, rproj};
+    for (uint32_t c0 = 0; c0 < nCols; c0 += 4) {
+        uint32_t const c = c0 + w;
+        bool const have = c < nCols;
+        double const cr = have ? src0[size_t(c) * 128] : 0.0, ci = have ? src0[size_t(c) * 128 + 64] : 0.0;
+        if (have && lane < 12)
+            hermite_1d<double>(H[w], x2[w], lane, L, image_pos + 4 * size_t(img), col_pos + 4 * size_t(c), hgrid);
+        __syncthreads();
+        if (have) {
+            float const d2z = x2[w][2][lane >> 4] - R2;
+            float const d2yz = x2[w][1][(lane >> 2) & 3] + d2z;
+            bool const in = (d2z < 0) && (d2yz < 0) && (x2[w][0][lane & 3] + d2yz < 0);
+            A[w][0][lane] = in ? cr : 0.0;
+            A[w][1][lane] = in ? ci : 0.0;
         }
-        hr = wave_sum(hr);
-        sr = wave_sum(sr);
-        if (j == 0) {
-            gmat[atom_mat_off[a] + size_t(k) * nc + l] = hr;
-            gmat[atom_mat_off[a] + size_t(nc) * nc + size_t(k) * nc + l] = sr;
+        __syncthreads();
+        if (have) {
+            for (int q = 0; q < nq; ++q) {
+                double const* Hx = H[w][jx[q]][0];
+                double const* Hy = H[w][jy[q]][1];
+                double const* Hz = H[w][jz[q]][2];
+                double const x0 = Hx[0], x1 = Hx[1], x2_ = Hx[2], x3 = Hx[3];
+#pragma unroll
+                for (int p = 0; p < 2; ++p) {
+                    double acc = 0;
+#pragma unroll
+                    for (int z = 0; z < 4; ++z) {
+                        double by = 0;
+#pragma unroll
+                        for (int y = 0; y < 4; ++y) {
+                            double const* r = &A[w][p][z * 16 + y * 4];
+                            by += Hy[y] * (((r[0] * x0 + r[1] * x1) + r[2] * x2_) + r[3] * x3);
+                        }
+                        acc += Hz[z] * by;
+                    }
+                    if (p == 0) sre[q] += acc; else sim[q] += acc;
+                }
+            }
         }
+        __syncthreads();   // A, H and x2 are free
+    }
+    for (int q = 0; q < nq; ++q) { part[w][0][lane + 64 * q] = sre[q]; part[w][1][lane + 64 * q] = sim[q]; }
+    __syncthreads();
+    if (tid < nc) {
+        double const re = (part[0][0][tid] + part[1][0][tid]) + (part[2][0][tid] + part[3][0][tid]);
+        double const im = (part[0][1][tid] + part[1][1][tid]) + (part[2][1][tid] + part[3][1][tid]);
+        double const pr = image_phase[2 * size_t(img)], pi = image_phase[2 * size_t(img) + 1];
+        uint64_t const off = uint64_t(desc[3 * size_t(img) + 1]) | uint64_t(desc[3 * size_t(img) + 2]) << 32;
+        D[off + size_t(i) * nc + tid] = (re * pi + im * pr) * factor;
     }
 }
 
@@ -2373,7 +2466,7 @@ template int device_autotune<double>(DevicePlan&, ActionScalars const&, double*,
 template int device_autotune<float>(DevicePlan&, ActionScalars const&, float*, float const*, hipStream_t, int, double*, std::string&);
 
 // The adjoint gradient (FP64): X solves (H - E_c S) X = B, Lam solves (H - conj(E_c) S) Lam = B column group by
-// column group; wE[c] = {w_c, -E_c w_c}.  Results on the host: gcell_host[ncell][64] (dL/dV per cell point) and
+// column group; wE[c] = {w_c, -E_c w_c}.  Results on the host: grad_V (dL/dV on the grid, unless null) and
 // gmat_host at atom_mat_off (per contributing atom [2][nc][nc], the derivative with respect to the entries of
 // (h dVol-scaled, s dVol-scaled) before the SHO prefactors, see gfa_gradient).
 // projection of one FP64 vector onto every atom image and collection per (atom, column group) with the Bloch
@@ -2407,21 +2500,43 @@ static int project_collect(DevicePlan& d, ActionScalars const& s, double const* 
     return 0;
 }
 
-int device_atom_coefficients(DevicePlan& d, ActionScalars const& s, double const* X, std::vector<double>& host,
-                             hipStream_t stream, std::string& err) {
-    size_t const n = size_t(d.ncoeffs) * d.nCols * 128;
-    host.assign(n, 0.0);
-    if (d.nAtoms == 0 || d.nchunks == 0 || n == 0) return 0;
-    if (!d.atom_coef)   // kept with the plan, like the other work buffers
-        if (int r = dalloc(d, d.atom_coef, n, err)) return r;
+int device_density_matrices(DevicePlan& d, Plan const& p, ActionScalars const& s, double const* X, double factor,
+                            double* D, hipStream_t stream, std::string& err) {
+    auto& w = d.dens;
+    if (!w.desc) {   // kept with the plan, like the other work buffers
+        std::vector<uint64_t> off(size_t(p.nAtoms) + 1, 0);
+        for (uint32_t a = 0; a < p.nAtoms; ++a) off[a + 1] = off[a] + uint64_t(nsho(p.atom_lmax[a])) * nsho(p.atom_lmax[a]);
+        w.n = off.back();
+        std::vector<uint32_t> desc(size_t(p.nAtomImages) * 3 + p.col_pos.size());
+        for (uint32_t i = 0; i < p.nAtomImages; ++i) {
+            uint32_t const a = p.image_atom[i];
+            desc[3 * size_t(i)] = p.atom_starts[a];
+            desc[3 * size_t(i) + 1] = uint32_t(off[a]);
+            desc[3 * size_t(i) + 2] = uint32_t(off[a] >> 32);
+        }
+        std::memcpy(desc.data() + size_t(p.nAtomImages) * 3, p.col_pos.data(), p.col_pos.size() * sizeof(float));
+        if (!d.atom_coef)
+            if (int r = dalloc(d, d.atom_coef, std::max<size_t>(1, size_t(d.ncoeffs) * d.nCols * 128), err)) return r;
+        if (!w.D)
+            if (int r = dalloc(d, w.D, std::max<size_t>(1, w.n), err)) return r;
+        if (int r = dupload(d, w.desc, desc, err)) return r;
+    }
+    if (d.nAtoms == 0 || d.nchunks == 0 || w.n == 0) {
+        std::fill(D, D + w.n, 0.0);
+        return 0;
+    }
     if (int r = project_collect(d, s, X, d.atom_coef, stream, err)) return r;
-    HIP_TRY(hipMemcpyAsync(host.data(), d.atom_coef, n * sizeof(double), hipMemcpyDeviceToHost, stream));
+    hipLaunchKernelGGL(k_density, dim3(d.nAtomImages, d.max_atom_nc), dim3(256), 0, stream, w.D, d.atom_coef, d.image_pos,
+                       d.image_lmax, d.image_phase, w.desc, d.nAtomImages, d.nCols, s.hgrid[0], s.hgrid[1], s.hgrid[2],
+                       s.hgrid[3], factor);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipMemcpyAsync(D, w.D, size_t(w.n) * sizeof(double), hipMemcpyDeviceToHost, stream));
     HIP_TRY(hipStreamSynchronize(stream));
     return 0;
 }
 
 int device_gradient(DevicePlan& d, Plan const& p, ActionScalars const& s, double const* X, double const* Lam,
-                    std::vector<double> const& wE, std::vector<double>& gcell_host, std::vector<double>& gmat_host,
+                    std::vector<double> const& wE, double* grad_V, std::vector<double>& gmat_host,
                     hipStream_t stream, std::string& err) {
     auto& g = d.grad;
     if (!g.ready) {
@@ -2448,18 +2563,18 @@ int device_gradient(DevicePlan& d, Plan const& p, ActionScalars const& s, double
     hipLaunchKernelGGL(k_grad_v_blocks, dim3(uint32_t(p.nnzb)), dim3(256), 0, stream, g.gpart, X, Lam, d.colindx,
                        d.veff, g.wE);
     hipLaunchKernelGGL(k_grad_v_cells, dim3(uint32_t(p.ncell())), dim3(64), 0, stream, g.gcell, g.gpart, g.cell_start,
-                       g.cell_blocks);
+                       g.cell_blocks, uint32_t(p.nb[0]), uint32_t(p.nb[1]));
     HIP_TRY(hipGetLastError());
     if (d.nAtoms > 0 && d.nchunks > 0) {
         for (int v = 0; v < 2; ++v)
             if (int r = project_collect(d, s, v ? Lam : X, v ? g.cL : g.cX, stream, err)) return r;
-        hipLaunchKernelGGL(k_grad_atoms, dim3(d.nAtoms, d.max_atom_nc), dim3(64), 0, stream, g.gmat, g.cX, g.cL,
+        hipLaunchKernelGGL(k_grad_atoms, dim3(d.nAtoms, d.max_atom_nc, (d.max_atom_nc + 3) / 4), dim3(256), 0, stream, g.gmat, g.cX, g.cL,
                            d.atom_lmax, d.atom_starts, d.atom_mat_off, g.wE, d.nCols);
         HIP_TRY(hipGetLastError());
     }
-    gcell_host.assign(size_t(p.ncell()) * 64, 0.0);
     gmat_host.assign(p.atom_mat_off.back(), 0.0);
-    HIP_TRY(hipMemcpyAsync(gcell_host.data(), g.gcell, gcell_host.size() * sizeof(double), hipMemcpyDeviceToHost, stream));
+    if (grad_V)   // (on a stream of its own, beside the kernels above, 691 -> 594 us in all; but creating one costs ms)
+        HIP_TRY(hipMemcpyAsync(grad_V, g.gcell, size_t(p.ncell()) * 64 * sizeof(double), hipMemcpyDeviceToHost, stream));
     if (d.nAtoms > 0 && d.nchunks > 0 && !gmat_host.empty())
         HIP_TRY(hipMemcpyAsync(gmat_host.data(), g.gmat, gmat_host.size() * sizeof(double), hipMemcpyDeviceToHost, stream));
     HIP_TRY(hipStreamSynchronize(stream));

@@ -344,76 +344,9 @@ int gfa_atom_density_matrices(gfa_plan* plan, const void* X, double factor, doub
             return fail(GFA_ERR_ARGUMENT, "atomic density matrices need one image per atom: the reduction over periodic "
                                           "images is not defined (include/green_dyadic.hxx:1085 asserts the same)");
         if (int s = ensure_device(plan)) return s;
-        std::vector<double> cx;
         std::string err;
-        if (gfa::device_atom_coefficients(plan->dev, scalars(h), (double const*)X, cx, (hipStream_t)stream, err))
+        if (gfa::device_density_matrices(plan->dev, h, scalars(h), (double const*)X, factor, D, (hipStream_t)stream, err))
             return fail(GFA_ERR_DEVICE, err);
-        std::vector<size_t> off(h.nAtoms + 1, 0);
-        for (uint32_t a = 0; a < h.nAtoms; ++a) off[a + 1] = off[a] + size_t(gfa::nsho(h.atom_lmax[a])) * gfa::nsho(h.atom_lmax[a]);
-        std::fill(D, D + off[h.nAtoms], 0.0);
-        typedef std::complex<double> cplx;
-        float const R2 = float(h.r_proj * h.r_proj);
-        for (uint32_t iai = 0; iai < h.nAtomImages; ++iai) {   // SHOprj_right (include/green_dyadic.hxx:925-1036)
-            int const L = h.image_lmax[iai];
-            int const nc = gfa::nsho(L), n2 = ((L + 1) * (L + 2)) / 2;
-            uint32_t const a = h.image_atom[iai], a0 = h.atom_starts[a];
-            double const* apos = &h.image_pos[4 * size_t(iai)];
-            double const sig_inv = apos[3] * apos[3];
-            // Hermite functions of this image at the 4x4x4 points of every source block: H[c][nu][dir][i4], the
-            // 1D functions of hermite_1d (include/green_dyadic.hxx:33-107) evaluated on the host
-            std::vector<double> H(size_t(h.nCols) * (L + 1) * 12);
-            std::vector<float> x2(size_t(h.nCols) * 12);
-            for (uint32_t c = 0; c < h.nCols; ++c)
-                for (int dir = 0; dir < 3; ++dir)
-                    for (int i4 = 0; i4 < 4; ++i4) {
-                        double const xi = sig_inv * ((double(h.col_pos[4 * c + dir]) * 4 + i4 + 0.5) * h.hg[dir] - apos[dir]);
-                        double const xx = xi * xi;
-                        x2[c * 12 + dir * 4 + i4] = float(xx);
-                        double hn = (xx < h.r_proj * h.r_proj) ? std::exp(-0.5 * xx) : 0.0, hm = 0;
-                        H[(c * (L + 1) + 0) * 12 + dir * 4 + i4] = hn;
-                        for (int nu = 0; nu < L; ++nu) {
-                            double const hp = xi * hn - (0.5 * nu) * hm;
-                            H[(c * (L + 1) + nu + 1) * 12 + dir * 4 + i4] = hp;
-                            hm = hn; hn = hp;
-                        }
-                    }
-            std::vector<cplx> piGp(size_t(nc) * nc, 0.0), czyx(nc), byx(n2), ax(L + 1);
-            for (int isho = 0; isho < nc; ++isho) {
-                std::fill(czyx.begin(), czyx.end(), cplx(0));
-                for (uint32_t c = 0; c < h.nCols; ++c) {
-                    double const* src = &cx[((size_t(a0) + isho) * h.nCols + c) * 128];
-                    auto Hc = [&](int nu, int dir, int i4) { return H[(c * (L + 1) + nu) * 12 + dir * 4 + i4]; };
-                    for (int z4 = 0; z4 < 4; ++z4) {
-                        float const d2z = x2[c * 12 + 8 + z4] - R2;
-                        if (!(d2z < 0)) continue;
-                        std::fill(byx.begin(), byx.end(), cplx(0));
-                        for (int y4 = 0; y4 < 4; ++y4) {
-                            float const d2yz = x2[c * 12 + 4 + y4] + d2z;
-                            if (!(d2yz < 0)) continue;
-                            std::fill(ax.begin(), ax.end(), cplx(0));
-                            for (int x4 = 0; x4 < 4; ++x4) {
-                                if (!(x2[c * 12 + x4] + d2yz < 0)) continue;
-                                int const xyz = (z4 * 4 + y4) * 4 + x4;
-                                cplx const pG(src[xyz], src[64 + xyz]);
-                                for (int ix = 0; ix <= L; ++ix) ax[ix] += pG * Hc(ix, 0, x4);
-                            }
-                            for (int iy = 0; iy <= L; ++iy) {
-                                int const iyx0 = (iy * (2 * L + 3 - iy)) >> 1;
-                                for (int ix = 0; ix <= L - iy; ++ix) byx[iyx0 + ix] += ax[ix] * Hc(iy, 1, y4);
-                            }
-                        }
-                        for (int jsho = 0, iz = 0; iz <= L; ++iz)
-                            for (int iy = 0; iy <= L - iz; ++iy) {
-                                int const iyx0 = (iy * (2 * L + 3 - iy)) >> 1;
-                                for (int ix = 0; ix <= L - iz - iy; ++ix) czyx[jsho++] += byx[iyx0 + ix] * Hc(iz, 2, z4);
-                            }
-                    }
-                }
-                for (int jsho = 0; jsho < nc; ++jsho) piGp[size_t(isho) * nc + jsho] = czyx[jsho];
-            }
-            cplx const ph(h.image_phase[2 * iai], h.image_phase[2 * iai + 1]);
-            for (size_t ij = 0; ij < piGp.size(); ++ij) D[off[a] + ij] += (piGp[ij] * ph).imag() * factor;
-        }
         return GFA_OK;
     });
 }
@@ -431,24 +364,12 @@ int gfa_gradient(gfa_plan* plan, const void* X, const void* Lambda, const double
             wE[4 * c] = wr; wE[4 * c + 1] = wi;
             wE[4 * c + 2] = -(er * wr - ei * wi); wE[4 * c + 3] = -(er * wi + ei * wr);   // -E w
         }
-        std::vector<double> gcell, gmat;
+        std::vector<double> gmat;
         std::string err;
         auto const sc = scalars(h);
-        if (gfa::device_gradient(plan->dev, h, sc, (double const*)X, (double const*)Lambda, wE, gcell, gmat,
+        if (gfa::device_gradient(plan->dev, h, sc, (double const*)X, (double const*)Lambda, wE, grad_V, gmat,
                                  (hipStream_t)stream, err))
             return fail(GFA_ERR_DEVICE, err);
-        if (grad_V) {   // cell-blocked -> grid [ng_z][ng_y][ng_x] (the inverse of gfa_set_potential's blocking)
-            size_t const ngx = 4 * size_t(h.nb[0]), ngy = 4 * size_t(h.nb[1]);
-            for (uint32_t bz = 0; bz < h.nb[2]; ++bz)
-            for (uint32_t by = 0; by < h.nb[1]; ++by)
-            for (uint32_t bx = 0; bx < h.nb[0]; ++bx) {
-                double const* src = &gcell[((size_t(bz) * h.nb[1] + by) * h.nb[0] + bx) * 64];
-                for (int z = 0; z < 4; ++z)
-                    for (int y = 0; y < 4; ++y)
-                        for (int x = 0; x < 4; ++x)
-                            grad_V[((bz * 4 + z) * ngy + (by * 4 + y)) * ngx + (bx * 4 + x)] = src[(z * 4 + y) * 4 + x];
-            }
-        }
         if (grad_hs) {  // per original atom [2][nc][nc]: dL/dh and dL/ds of the matrices given to gfa_set_atom_matrices
             size_t const natoms = h.xyzZinso.size() / 8;
             std::vector<size_t> off(natoms + 1, 0);

@@ -33,11 +33,17 @@ struct GradWs {  // buffers of the adjoint gradient
     uint32_t* cell_start = nullptr;   // [ncell+1] blocks reading each cell block's potential
     uint32_t* cell_blocks = nullptr;
     double* gpart = nullptr;          // [nnzb][64]
-    double* gcell = nullptr;          // [ncell][64]
+    double* gcell = nullptr;          // [ncell * 64] on the grid [4 nbz][4 nby][4 nbx]
     double* wE = nullptr;             // [nCols][4]: w_c, -E_c w_c
     double* cX = nullptr;             // [ncoeffs][nCols][2][64] collected atom coefficients of X
     double* cL = nullptr;             // same for lambda
     double* gmat = nullptr;           // per contributing atom [2][nc][nc]
+};
+
+struct DensWs {  // buffers of the atomic density matrices
+    uint32_t* desc = nullptr;         // [nai][3] coefficient row and matrix offset of its atom, then col_pos
+    double* D = nullptr;              // [n] the matrices
+    uint64_t n = 0;
 };
 
 struct DevicePlan {
@@ -119,6 +125,7 @@ struct DevicePlan {
 
     Workspace<double> ws64;
     GradWs grad;
+    DensWs dens;
     double* atom_coef = nullptr;       // [ncoeffs][nCols][2][64] atom projections (density matrices)
     Workspace<float> ws32;
     size_t bytes = 0;
@@ -161,12 +168,12 @@ int device_action_noalloc(DevicePlan& d, ActionScalars const& s, real_t* y, real
 template <typename real_t>
 int device_autotune(DevicePlan& d, ActionScalars const& s, real_t* y, real_t const* x, hipStream_t stream, int reps,
                     double* best_ms, std::string& err);
-// the projections of an FP64 vector X onto every atom, collected over its images with the Bloch phases, on the
-// host: [((atom_starts[a] + s) * nCols + c)][re/im][j]
-int device_atom_coefficients(DevicePlan& d, ActionScalars const& s, double const* X, std::vector<double>& host,
-                             hipStream_t stream, std::string& err);
+// atomic density matrices of an FP64 vector X into D on the host (per contributing atom [nc][nc]); every atom has one
+// image
+int device_density_matrices(DevicePlan& d, Plan const& p, ActionScalars const& s, double const* X, double factor,
+                            double* D, hipStream_t stream, std::string& err);
 int device_gradient(DevicePlan& d, Plan const& p, ActionScalars const& s, double const* X, double const* Lam,
-                    std::vector<double> const& wE, std::vector<double>& gcell_host, std::vector<double>& gmat_host,
+                    std::vector<double> const& wE, double* grad_V, std::vector<double>& gmat_host,
                     hipStream_t stream, std::string& err);
 double reference_flops(Plan const& p, int fp_bits);
 
