@@ -299,17 +299,18 @@ __global__ __launch_bounds__(256) void k_sho_project_mfma(
 // ---------------------------------------------------------------------------------------------
 // 2. per (atom, column): collect images with phase, multiply (h - E s) dVol, broadcast with conjugate phase.
 //    The 64 right-hand sides of a column group are independent, so a work-group takes JS of them for one (atom,
-//    column): 512 threads collect the chunk partial sums into LDS (thread = one right-hand side of one coefficient,
-//    both planes), then the waves multiply on the matrix cores.  h and s are real, so with the collected c = (c_re,
+//    column): 1,024 threads collect the chunk partial sums into LDS (thread = one right-hand side of one coefficient,
+//    both planes, and where few coefficients leave threads over, one of P parts of the chunk list), then the waves multiply on the matrix cores.  h and s are real, so with the collected c = (c_re,
 //    c_im) the products t = h c and u = s c are real contractions, [16 rows of h and s] x [nc] x [16 right-hand sides
 //    of both planes] per wave on the FP64 16x16x4 MFMA (operand layout as in k_sho_project_mfma), and d = t - E u.
 //    Bound by latency: a plan has few (atom, column) pairs, and one pair's chain (chunk list, partial sums, matrix)
 //    is what a launch takes.  The chunks of a pair are therefore one list in memory, read ahead of the sums, the
-//    first 64 columns of the wave's matrix rows are loaded before the collection, and JS is small enough for four
-//    (two) work-groups per pair.  Measured, against one work-group of 8 waves per pair on the vector ALUs that read
-//    chunk by chunk: FP64 numax 5, 215 pairs: 212 -> 73 us; numax 7, 16 pairs: 428 -> 46 us; numax 2, 2 pairs of 13
-//    images: 63 -> 19 us; FP32 numax 5, 1,370 pairs: 309 -> 164 us.  Holding the kernel to 128 VGPRs (4 waves per
-//    SIMD instead of 3) spills and takes 96, 55, 22 and 225 us.
+//    wave's first matrix columns are loaded before the collection, and JS is small enough for four (two) work-groups
+//    per pair.  Measured, against one work-group of 8 waves per pair on the vector ALUs that read chunk by chunk, then
+//    with 512 threads without parts, then as it is: FP64 numax 5, 215 pairs: 212, 79, 79 us; numax 7, 16 pairs: 428, 47,
+//    42 us; numax 2, 2 pairs of 13 images: 63, 16, 13 us; numax 3, 4 pairs: 18 -> 15 us; FP32 numax 5, 1,370 pairs:
+//    309, 187, 157 us.  P follows from the coefficients alone (and the precision), so that a pair's sum has the same
+//    order in every plan.  KA = 4 keeps 1,024 threads within 128 VGPRs with all of the parts' loads (8: the same times).
 // ---------------------------------------------------------------------------------------------
 // one chunk of the projection partial sums of an (atom, column): its first coefficient row and its atom image
 struct CollectEntry {
@@ -353,7 +354,7 @@ __device__ __forceinline__ void collect_coefficient(real_t const* __restrict__ p
     if (e < e1) collect_chunks<real_t, 8>(partial, coll, e, e1, image_phase, s, j, ar, ai);
 }
 
-constexpr int ATOM_T = 512;   // threads of k_sho_atoms
+constexpr int ATOM_T = 1024;   // threads of k_sho_atoms
 
 template <typename real_t, int JS>
 __global__ __launch_bounds__(ATOM_T) void k_sho_atoms(
@@ -366,7 +367,7 @@ __global__ __launch_bounds__(ATOM_T) void k_sho_atoms(
     double const* __restrict__ E_col, uint8_t const* __restrict__ col_active) {
     using acc_t = typename Mfma<double>::acc_t;
     constexpr int NS = 64 / JS, NJ = JS / 16;   // slices per pair, 16-column tiles per plane
-    constexpr int KA = 16;                      // k-steps (of 4 columns of h and s) loaded together
+    constexpr int KA = 4;                       // k-steps (of 4 columns of h and s) loaded together
     extern __shared__ double cs[];              // [plane][16-column tile][coefficient, padded to 4][16]
     // the pairs with a block of the column near the atom: those of small truncation spheres see few of the atoms,
     // and the coefficients of the others are never read
@@ -395,14 +396,30 @@ __global__ __launch_bounds__(ATOM_T) void k_sho_atoms(
     };
     if (w < nu) load_rows(w / NJ, 0);
 
-    for (int s = tid / JS; s < kp; s += ATOM_T / JS) {
-        int const jl = tid % JS;
+    // few coefficients: the threads take P parts of the chunk list, summed in part order below
+    constexpr int SLOTS = ATOM_T / (sizeof(real_t) == 8 ? 16 : 32);
+    int P = 1;
+    while (2 * P * kp <= SLOTS) P *= 2;
+    uint32_t const per = (e1 - e0 + P - 1) / P;
+    int const jl = tid % JS;
+    for (int t = tid / JS; t < P * kp; t += ATOM_T / JS) {
+        int const part = __builtin_amdgcn_readfirstlane(t / kp), s = t - part * kp;   // kp and the wave: multiples of 4
+        uint32_t const p0 = min(e0 + part * per, e1), p1 = min(p0 + per, e1);
         double ar = 0, ai = 0;
-        if (s < nc) collect_coefficient<real_t>(partial, coll, e0, e1, image_phase, s, slice * JS + jl, ar, ai);
-        cs[((jl >> 4) * kp + s) * 16 + (jl & 15)] = ar;
-        cs[((NJ + (jl >> 4)) * kp + s) * 16 + (jl & 15)] = ai;
+        if (s < nc) collect_coefficient<real_t>(partial, coll, p0, p1, image_phase, s, slice * JS + jl, ar, ai);
+        double* dst = cs + (size_t(part) * 2 * NJ * kp + (jl >> 4) * kp + s) * 16 + (jl & 15);
+        dst[0] = ar;
+        dst[NJ * kp * 16] = ai;
     }
     __syncthreads();
+    if (P > 1) {
+        for (int t = tid; t < 2 * JS * kp; t += ATOM_T) {
+            double v = cs[t];
+            for (int part = 1; part < P; ++part) v += cs[part * 2 * JS * kp + t];
+            cs[t] = v;
+        }
+        __syncthreads();
+    }
 
     uint32_t const k0 = sum_start[a], k1 = sum_start[a + 1];
     for (int u = w; u < nu; u += ATOM_T / 64) {
@@ -2236,7 +2253,7 @@ int device_action(DevicePlan& d, ActionScalars const& s, real_t* y, real_t const
         uint64_t const pairs = d.n_atom_pairs;
         int const JS = (sizeof(real_t) == 4 && pairs >= 512) ? 32 : 16;
         if (pairs * (64 / JS) > 0x7fffffffull) { err = "too many (atom, column) pairs for one launch"; return 1; }
-        size_t const lds = size_t(2) * JS * ((d.max_atom_nc + 3) & ~3u) * sizeof(double);
+        size_t const lds = size_t(2) * JS * std::max<size_t>((d.max_atom_nc + 3) & ~3u, ATOM_T / 16) * sizeof(double);
 #define LAUNCH_ATOMS(JS_) hipLaunchKernelGGL((k_sho_atoms<real_t, JS_>), dim3(uint32_t(pairs) * (64 / JS_)), \
             dim3(ATOM_T), lds, stream, ws.dcoef, ws.partial, d.atom_pairs, d.coll_start, \
             reinterpret_cast<CollectEntry const*>(d.coll), d.sum_start, d.sum_index, d.image_starts, d.atom_lmax, d.atom_hs, d.atom_mat_off, d.image_phase, d.nCols, \
