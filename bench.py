@@ -42,7 +42,7 @@ TRAFFIC_FILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profile
 # MFMA utilisation of the matrix-core forms of the SHO projection and add-back on this workload (rocprofv3
 # SQ_VALU_MFMA_BUSY_CYCLES, SQ_INSTS_VALU_MFMA_MOPS_* of --mode dyadic); the commands are in the file
 MFMA_FILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles", "dyadic_mfma_contour32_counters.json")
-KERNEL_OF_KIND = {0: "k_local", 1: "k_plane", 2: "k_lines"}
+KERNEL_OF_KIND = {0: "k_local", 1: "k_plane", 2: "k_lines"}   # FP32, 8th order: (1, 32, 0) is run by k_lines
 SOURCE = (16, 16, 16)
 NBATCH = 4
 
@@ -366,7 +366,7 @@ def main():
         "roofline": {"bound": "hbm", "achieved": round(alg32 / t_loc32 / 1e9, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(alg32 / t_loc32 / 1e9 / HBM_PEAK_GBS, 4),
                      "traffic": traffic_of(shape32, nnzb),
-                     "kernel": f"FP32 local kernel, tile shape {shape32} ({KERNEL_OF_KIND.get(shape32[0])}: "
+                     "kernel": f"FP32 local kernel, tile shape {shape32} ({'k_lines' if tuple(shape32[:2]) == (1, 32) else KERNEL_OF_KIND.get(shape32[0])}: "
                                "potential + 8th-order kinetic + SHO add-back), the one the mixed solve ran, on the "
                                "batch-0 plan; algorithmic bytes per launch = nnzb * 2 * 32 KiB + nRows * 512 B"},
         "cpu_baseline": cpu,
