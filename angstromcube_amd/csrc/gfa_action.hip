@@ -1744,6 +1744,16 @@ int device_upload_plan(Plan const& p, DevicePlan& d, std::string& err) {
         d.fd_range[dd] = p.kinetic[dd].fd_range;
         if (p.kinetic[dd].fd_range == 8) d.nh_max = 2;
     }
+    if (!d.tuned[1]) {
+        // the FP32 default shape.  Up to the 8th order k_lines, 32 columns, 2 directions ahead: it adds the images in
+        // the plane form of k_plane but reads and writes 16 bytes per lane (against k_plane with 32 columns: 158,112
+        // blocks 3,347 us against 3,779, 19,764 blocks 424 against 472, 1,461 blocks 31.1 against 35.2, 6,144 blocks
+        // with images 138 against 156, 64 blocks 15.0 against 16.6).  With a direction of the 16th order k_local, 32
+        // columns, whose registers hold two lines instead of a plane or a direction (against k_plane: 3,246 blocks 91.5
+        // us against 106, 22,948 blocks 765 against 915; mixed orders with images, 4,096 blocks 133 against 383)
+        bool const wide = d.nh_max == 2;
+        d.tune_kind[1] = wide ? 0 : 2; d.tune_jw[1] = 32; d.tune_lb[1] = 2;
+    }
     int s = 0;
     if ((s = dupload(d, d.colindx, p.colindx, err))) return s;
     if ((s = dupload(d, d.rowindx, p.rowindx, err))) return s;
@@ -2158,11 +2168,7 @@ __global__ __launch_bounds__(256) void k_density(double* __restrict__ D, double 
 }
 
 // Local-kernel tile shapes.  kind 0: k_local (LDS accumulator), JW columns per work-group (16 or 32), LB
-// kinetic lines per thread in flight (1, 2, 4).  kind 1: k_plane (register accumulator), JW = 32 or 64; its FP32
-// 8th-order shape of 32 columns, the default, is run by k_lines with 2 directions ahead, which adds the images in
-// the same plane form but reads and writes 16 bytes per lane: 158,112 blocks 3,347 us against 3,779 for k_plane,
-// 19,764 blocks 424 against 472, 1,461 blocks 31.1 against 35.2, 6,144 blocks with images 138 against 156, 64 blocks
-// 15.0 against 16.6.
+// kinetic lines per thread in flight (1, 2, 4).  kind 1: k_plane (register accumulator), JW = 32 or 64.
 // kind 2: k_lines (16-byte lanes, line ownership), JW = 16 or 32, or 64 in FP32; LB = directions of neighbour
 // lines issued up front (3 or 2; 16th-order stencils issue one direction at a time).
 template <typename real_t, int NH, bool IMG>
@@ -2185,9 +2191,7 @@ static void launch_local(int kind, int jw, int lb, dim3 g, hipStream_t stream, L
             else KN(32, 3);
         }
     } else if (kind == 1) {
-        if (jw == 64) KP(64);
-        else if constexpr (sizeof(real_t) == 4 && NH == 1) KN(32, 2);   // the faster kernel on every plan measured
-        else KP(32);
+        if (jw == 64) KP(64); else KP(32);
     } else if (jw == 16) {
         if (lb == 1) KL(16, 1); else if (lb == 4) KL(16, 4); else KL(16, 2);
     } else {

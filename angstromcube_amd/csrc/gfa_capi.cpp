@@ -127,10 +127,6 @@ int gfa_plan_create(const gfa_plan_desc* desc, gfa_plan** plan) {
             delete p;
             return fail(GFA_ERR_ARGUMENT, err);
         }
-        // FP32 local kernel of the 16th-order stencil: the LDS accumulator, whose registers hold two lines instead of a
-        // plane (3,180 blocks: 105 us against 112 for k_plane; 22,948 blocks: 765 against 915)
-        for (int d = 0; d < 3; ++d)
-            if (p->host.kinetic[d].fd_range == 8) { p->dev.tune_kind[1] = 0; p->dev.tune_lb[1] = 2; }
         if (p->echo > 0)
             std::printf("# gfa plan: %u rows, %u columns, %llu blocks, %u atoms, %u images\n", p->host.nRows,
                         p->host.nCols, (unsigned long long)p->host.nnzb, p->host.nAtoms, p->host.nAtomImages);

@@ -54,9 +54,9 @@ struct DevicePlan {
     int nh_max = 1;                    // neighbour blocks per side in the widest stencil
     bool has_images = false;           // some finite-difference halo is a periodic image
     int fd_range[3] = {4, 4, 4};
-    // local-kernel tile shape per precision (index 0: FP64, 1: FP32), set by the autotuner; the defaults are the
-    // shapes measured fastest: k_lines, 2 directions ahead, with 16 columns in FP64 and 32 in FP32 (under kind 1, see
-    // launch_local)
+    // local-kernel tile shape per precision (index 0: FP64, 1: FP32), pinned or set by the autotuner (tuned); the
+    // defaults are the shapes measured fastest, in FP64 k_lines with 16 columns, 2 directions ahead, in FP32 by the
+    // stencil's order when the plan goes to the device (device_upload_plan)
     int tune_kind[2] = {2, 1}, tune_jw[2] = {16, 32}, tune_lb[2] = {2, 0};
     bool tuned[2] = {false, false};
     // SHO projection and add-back per precision: 0 the sum-factorised forms on the vector ALUs (the add-back inside

@@ -42,7 +42,7 @@ TRAFFIC_FILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profile
 # MFMA utilisation of the matrix-core forms of the SHO projection and add-back on this workload (rocprofv3
 # SQ_VALU_MFMA_BUSY_CYCLES, SQ_INSTS_VALU_MFMA_MOPS_* of --mode dyadic); the commands are in the file
 MFMA_FILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles", "dyadic_mfma_contour32_counters.json")
-KERNEL_OF_KIND = {0: "k_local", 1: "k_plane", 2: "k_lines"}   # FP32, 8th order: (1, 32, 0) is run by k_lines
+KERNEL_OF_KIND = {0: "k_local", 1: "k_plane", 2: "k_lines"}
 SOURCE = (16, 16, 16)
 NBATCH = 4
 
@@ -366,7 +366,7 @@ def main():
         "roofline": {"bound": "hbm", "achieved": round(alg32 / t_loc32 / 1e9, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(alg32 / t_loc32 / 1e9 / HBM_PEAK_GBS, 4),
                      "traffic": traffic_of(shape32, nnzb),
-                     "kernel": f"FP32 local kernel, tile shape {shape32} ({'k_lines' if tuple(shape32[:2]) == (1, 32) else KERNEL_OF_KIND.get(shape32[0])}: "
+                     "kernel": f"FP32 local kernel, tile shape {shape32} ({KERNEL_OF_KIND.get(shape32[0])}: "
                                "potential + 8th-order kinetic + SHO add-back), the one the mixed solve ran, on the "
                                "batch-0 plan; algorithmic bytes per launch = nnzb * 2 * 32 KiB + nRows * 512 B"},
         "cpu_baseline": cpu,
@@ -391,7 +391,7 @@ def action_mode(G, sysm, instances, n, args, stream, dev):
         p.set_tile_shape(64, *shape)
         t = time_action(p, 64, 2, args.action_reps, stream)
         log(f"# local fp64 shape {shape}: {t * 1e3:.3f} ms for {p.nnzb} blocks")
-    p.set_tile_shape(32, 1, 32, 0)   # the default shapes again for the engine comparison
+    p.set_tile_shape(32, 2, 32, 2)   # the default shapes again for the engine comparison
     p.set_tile_shape(64, 2, 16, 2)
     dyadic_engines(p, args, stream)
     # a plain device copy of one FP64 vector (nnzb * 64 KiB each way): the calibration of HBM counters

@@ -170,8 +170,7 @@ int gfa_action_part(gfa_plan* plan, int fp_bits, int part, void* y, const void* 
  *      No counterpart in the reference, whose kernels have fixed launch shapes. ---- */
 int gfa_autotune(gfa_plan* plan, int fp_bits, void* y, const void* x, void* stream, int reps, double* best_ms);
 /* pins the tile shape instead: kind 0 (LDS accumulator): columns per work-group 16 or 32, kinetic lines per
- * thread in flight 1, 2 or 4; kind 1 (register accumulator per z plane): columns 32 or 64, lines ignored
- * (in FP32, for stencils up to the 8th order, 32 columns run as kind 2 with 2 lines, which is faster);
+ * thread in flight 1, 2 or 4; kind 1 (register accumulator per z plane): columns 32 or 64, lines ignored;
  * kind 2 (16-byte lanes, each thread owning one x-, y- and z-line): columns 16 or 32 (or 64 in FP32), lines = the
  * directions whose neighbour lines are loaded before the first stencil, 2 or 3 */
 int gfa_set_tile_shape(gfa_plan* plan, int fp_bits, int kind, int columns, int lines);
@@ -184,7 +183,9 @@ int gfa_set_tile_shape(gfa_plan* plan, int fp_bits, int kind, int columns, int l
 int gfa_set_dyadic_engine(gfa_plan* plan, int fp_bits, int engine);
 int gfa_get_dyadic_engine(gfa_plan* plan, int fp_bits, int* engine);
 /* the tile shape the action of fp_bits uses (the autotuner's choice, the pinned one or the default); *tuned = 1
- * when it was set by gfa_autotune or gfa_set_tile_shape */
+ * when it was set by gfa_autotune or gfa_set_tile_shape.  The FP32 default is settled when the plan goes to the device
+ * (gfa_plan_prepare or the first call that runs there): kind 2, 32 columns, 2 lines up to the 8th order, kind 0, 32
+ * columns, 2 lines with a direction of the 16th; before that a plan with no shape set reports kind 1, 32 columns */
 int gfa_get_tile_shape(gfa_plan* plan, int fp_bits, int* kind, int* columns, int* lines, int* tuned);
 
 /* ---- the solve (H - E S) X = B with B = unit columns on the diagonal blocks; replaces
