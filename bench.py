@@ -366,7 +366,7 @@ def main():
         "roofline": {"bound": "hbm", "achieved": round(alg32 / t_loc32 / 1e9, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(alg32 / t_loc32 / 1e9 / HBM_PEAK_GBS, 4),
                      "traffic": traffic_of(shape32, nnzb),
-                     "kernel": f"FP32 local kernel, tile shape {shape32} ({KERNEL_OF_KIND.get(shape32[0])}: "
+                     "kernel": f"FP32 local kernel, tile shape {shape32} ({fp32_kernel(shape32)}: "
                                "potential + 8th-order kinetic + SHO add-back), the one the mixed solve ran, on the "
                                "batch-0 plan; algorithmic bytes per launch = nnzb * 2 * 32 KiB + nRows * 512 B"},
         "cpu_baseline": cpu,
@@ -494,16 +494,23 @@ def contour_mode(G, sysm, args):
     print(json.dumps(out))
 
 
+def fp32_kernel(shape):
+    """The FP32 local kernel that a tile shape runs on this workload (8th order, no periodic images), as a profile
+    names it."""
+    kind, columns, lines = shape
+    return f"{KERNEL_OF_KIND[kind]}<float, 1, false, {columns}" + ("" if kind == 1 else f", {lines}") + ">"
+
+
 def traffic_of(shape, nnzb):
     """HBM bytes (read + written) per launch of the FP32 local kernel of this tile shape, from the committed
-    rocprofv3 counter summary of the same workload; None if it covers another workload or shape."""
+    rocprofv3 counter summary of the same workload; None if it covers another workload, shape or kernel."""
     try:
         with open(TRAFFIC_FILE) as f:
             t = json.load(f)
     except (OSError, ValueError):
         return None
     e = t.get("shapes", {}).get(",".join(str(v) for v in shape))
-    if t.get("nnzb") != int(nnzb) or e is None:
+    if t.get("nnzb") != int(nnzb) or e is None or e.get("kernel") != fp32_kernel(shape):
         return None
     return int(e["fetch_bytes"] + e["write_bytes"])
 
