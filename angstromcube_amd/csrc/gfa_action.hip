@@ -2334,8 +2334,8 @@ template int device_action<float>(DevicePlan&, ActionScalars const&, float*, flo
 
 // ---------------------------------------------------------------------------------------------
 // The action without allocation (gfa_action_noalloc): the projection partial sums, the addition coefficients
-// and the zero block live in `scratch`, a fixed array of every GPU the library runs on (held until the process ends).  Its device address is taken once per device with
-// hipGetSymbolAddress; the host-side name `scratch` is never handed to a kernel.  Calls that overlap on one GPU
+// and the zero block live in `scratch`, a fixed array of every GPU the library runs on (held until the process
+// ends).  Its device address is taken once per device with hipGetSymbolAddress; the host-side name `scratch` is never handed to a kernel.  Calls that overlap on one GPU
 // share the array and race.
 // ---------------------------------------------------------------------------------------------
 namespace {
@@ -2379,9 +2379,6 @@ size_t noalloc_scratch_bytes(DevicePlan const& d, int fp_bits) {
     if (d.nAtomImages > 0) {
         b += round256(size_t(d.total_chunk_coefs) * 128 * s);
         b += round256(size_t(d.natomcoeffs) * d.nCols * 128 * s);
-        // one FP64 row per collected coefficient of a plan with numax 6, 7 atoms: no longer stored, but the plans the
-        // allocation-free action takes stay the same
-        if (d.nchunks > 0 && d.max_atom_nc > 64) b += round256(size_t(d.ncoeffs) * d.nCols * 128 * 8);
     }
     return b;
 }
