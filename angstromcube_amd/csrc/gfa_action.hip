@@ -300,9 +300,10 @@ __global__ __launch_bounds__(256) void k_sho_project_mfma(
 // 2. per (atom, column): collect images with phase, multiply (h - E s) dVol, broadcast with conjugate phase.
 //    The 64 right-hand sides of a column group are independent, so a work-group takes JS of them for one (atom,
 //    column): 1,024 threads collect the chunk partial sums into LDS (thread = one right-hand side of one coefficient,
-//    both planes, and where few coefficients leave threads over, one of P parts of the chunk list), then the waves multiply on the matrix cores.  h and s are real, so with the collected c = (c_re,
-//    c_im) the products t = h c and u = s c are real contractions, [16 rows of h and s] x [nc] x [16 right-hand sides
-//    of both planes] per wave on the FP64 16x16x4 MFMA (operand layout as in k_sho_project_mfma), and d = t - E u.
+//    both planes, and where few coefficients leave threads over, one of P parts of the chunk list), then the waves
+//    multiply on the matrix cores.  h and s are real, so with the collected c = (c_re, c_im) the products t = h c and
+//    u = s c are real contractions, [16 rows of h and s] x [nc] x [16 right-hand sides of both planes] per wave on the
+//    FP64 16x16x4 MFMA (operand layout as in k_sho_project_mfma), and d = t - E u.
 //    Bound by latency: a plan has few (atom, column) pairs, and one pair's chain (chunk list, partial sums, matrix)
 //    is what a launch takes.  The chunks of a pair are therefore one list in memory, read ahead of the sums, the
 //    wave's first matrix columns are loaded before the collection, and JS is small enough for four (two) work-groups
@@ -2251,11 +2252,13 @@ int device_action(DevicePlan& d, ActionScalars const& s, real_t* y, real_t const
 #undef LAUNCH_MFMA
             HIP_TRY(hipGetLastError());
         }
-        // right-hand sides per work-group: 16 fill 128-byte lines in FP64; in FP32 32 do (1,370 pairs: 164 us
-        // against 182 us with 16), and 16 (twice the work-groups, half lines) are taken while 32 would leave CUs
-        // idle, below 512 pairs = 1,024 work-groups
+        // right-hand sides per work-group: 16 fill 128-byte lines in FP64; in FP32 32 do, and 16 (twice the work-groups,
+        // half lines) are taken while 32 would leave CUs without one, below 128 pairs = 256 work-groups.  Measured, FP32,
+        // 16 against 32: numax 7, 88 pairs 61 us against 73, 264 pairs 131 against 118, 704 pairs 251 against 215; numax 5,
+        // 140 pairs 46 against 38, 1,392 pairs 218 against 161; numax 3, 104 pairs 15.3 against 15.5, 312 pairs 34 against
+        // 24; numax 2, 104 pairs 12.6 against 11.5, 832 pairs 55 against 37
         uint64_t const pairs = d.n_atom_pairs;
-        int const JS = (sizeof(real_t) == 4 && pairs >= 512) ? 32 : 16;
+        int const JS = (sizeof(real_t) == 4 && pairs >= 128) ? 32 : 16;
         if (pairs * (64 / JS) > 0x7fffffffull) { err = "too many (atom, column) pairs for one launch"; return 1; }
         size_t const lds = size_t(2) * JS * std::max<size_t>((d.max_atom_nc + 3) & ~3u, ATOM_T / 16) * sizeof(double);
 #define LAUNCH_ATOMS(JS_) hipLaunchKernelGGL((k_sho_atoms<real_t, JS_>), dim3(uint32_t(pairs) * (64 / JS_)), \
