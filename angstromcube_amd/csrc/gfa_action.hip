@@ -310,8 +310,9 @@ __global__ __launch_bounds__(256) void k_sho_project_mfma(
 //    per pair.  Measured, against one work-group of 8 waves per pair on the vector ALUs that read chunk by chunk, then
 //    with 512 threads without parts, then as it is: FP64 numax 5, 215 pairs: 212, 79, 79 us; numax 7, 16 pairs: 428, 47,
 //    42 us; numax 2, 2 pairs of 13 images: 63, 16, 13 us; numax 3, 4 pairs: 18 -> 15 us; FP32 numax 5, 1,370 pairs:
-//    309, 187, 157 us.  P follows from the coefficients alone (and the precision), so that a pair's sum has the same
-//    order in every plan.  KA = 4 keeps 1,024 threads within 128 VGPRs with all of the parts' loads (8: the same times).
+//    309, 187, 157 us.  P follows from the coefficients (and the precision), not from JS, so that the order of a pair's
+//    sum follows from its chunk list alone; the length of the chunks follows from the whole plan (device_upload_plan),
+//    so between plans of different sizes a sum may differ by rounding.  KA = 4 keeps 1,024 threads within 128 VGPRs with all of the parts' loads (8: the same times).
 // ---------------------------------------------------------------------------------------------
 // one chunk of the projection partial sums of an (atom, column): its first coefficient row and its atom image
 struct CollectEntry {
@@ -613,8 +614,8 @@ __device__ __forceinline__ void sho_add_regs(real_t (&out)[16], real_t const (*H
 }
 
 // The images of a block's add list are taken in batches whose coefficients fit a buffer of CAP rows in LDS, so that a
-// work-group pays one round trip to memory and two barriers per batch: with numax 2 four images, numax 3 two, numax 4
-// and 5 one at a time.
+// work-group pays one round trip to memory and two barriers per batch: with numax 2 four images, numax 3 two (CAP 56) or
+// three (CAP 64), numax 4 and 5 one at a time.
 constexpr int BATCH = 4;
 template <typename real_t>
 struct BatchHermite { real_t H[BATCH][6][3][4]; };

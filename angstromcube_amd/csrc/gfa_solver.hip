@@ -48,8 +48,9 @@ constexpr int NBLK = 2 * 64 * 64;
 #define VEC_NT 1
 #endif
 // blocks per segment (work-group of the vector kernels) of a column group of n blocks: a power of two, at most 16, and
-// few enough for 1,024 segments.  It depends on the group alone, so that a group's sums, and with them its iterates, do
-// not depend on the other groups of the plan.  With 16 blocks whatever the group, 1,024 blocks made 64 work-groups and
+// few enough for 1,024 segments.  It depends on the group alone, so that the order of a group's sums over its blocks does
+// not depend on the other groups of the plan (the action's projection sums do, by the chunk length that follows from
+// the plan's size: between plans of different sizes iterates may differ by rounding).  With 16 blocks whatever the group, 1,024 blocks made 64 work-groups and
 // left three quarters of the CUs idle: FP64, 1,024 blocks: k_cocg_r 83 us against 29 with 1 block, k_cocg_px_odd 150
 // against 47; 1,461 blocks: k_dx2 348 against 117, k_even 160 against 85
 uint32_t segment_blocks(uint64_t n) {
