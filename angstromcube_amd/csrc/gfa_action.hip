@@ -121,21 +121,17 @@ template <typename real_t, int L>
 __global__ __launch_bounds__(128) void k_sho_project(
     real_t* __restrict__ partial, real_t const* __restrict__ x, ProjChunk const* __restrict__ chunks,
     uint32_t const* __restrict__ bucket, uint32_t const* __restrict__ chunk_coef,
-    uint32_t const* __restrict__ prj_blocks, uint32_t const* __restrict__ rowindx,
-    float const* __restrict__ row_pos, double const* __restrict__ image_pos, double hx, double hy, double hz,
-    double rproj, uint8_t const* __restrict__ col_active, double const* __restrict__ htab,
-    uint64_t const* __restrict__ smask, uint32_t const* __restrict__ prj_slot) {
+    uint32_t const* __restrict__ prj_blocks, uint8_t const* __restrict__ col_active,
+    double const* __restrict__ htab, uint64_t const* __restrict__ smask, uint32_t const* __restrict__ prj_slot) {
     __shared__ real_t H[L + 1][3][4];
     uint32_t const ich = bucket[blockIdx.x];
     ProjChunk const ch = chunks[ich];
     if (col_active && !col_active[ch.col]) return;  // a retired column group
     int const tid = threadIdx.x, j = tid & 63, p = tid >> 6;
-    (void)rowindx; (void)row_pos; (void)image_pos; (void)hx; (void)hy; (void)hz;
     constexpr int n3 = Sho<L>::n3, n2 = Sho<L>::n2;
     real_t czyx[n3];
 #pragma unroll
     for (int s = 0; s < n3; ++s) czyx[s] = 0;
-    (void)rproj;
     for (uint32_t b = ch.begin; b < ch.end; ++b) {
         uint32_t const inzb = prj_blocks[b];
         uint64_t const in = smask[prj_slot[b]];   // uniform
@@ -424,6 +420,8 @@ __global__ __launch_bounds__(ATOM_T) void k_sho_atoms(
     }
 
     uint32_t const k0 = sum_start[a], k1 = sum_start[a + 1];
+    // at most 8 * NJ = ATOM_T / 64 tiles: one per wave.  The loop has one turn, but as straight-line code, with its first
+    // load_rows no longer kept apart, the kernel is slower (FP32 numax 5, 1,370 pairs: by 6%; FP64 numax 7, 16 pairs: 5%)
     for (int u = w; u < nu; u += ATOM_T / 64) {
         int const mt = u / NJ, jt = u % NJ;
         acc_t tr = {0, 0, 0, 0}, ti = {0, 0, 0, 0}, ur = {0, 0, 0, 0}, ui = {0, 0, 0, 0};
@@ -523,7 +521,6 @@ struct LocalArgs {
     int nh[3];               // neighbour blocks per side used in direction d (1 or 2)
     real_t cdiag;            // sum of the centre weights of the three directions
     double phase[3][2][2];
-    double hgrid[4];
 };
 
 // sum over the SHO coefficients c[iz][iy][ix] (ix fastest, iz + iy + ix <= L) of one atom image at the 16
@@ -1321,7 +1318,7 @@ __device__ __forceinline__ void phase_lines(LocalArgs<real_t> const& a, int d, I
 // stencil; 1: x, then y after the x stencil and z after the y stencil) -- loads in flight against occupancy.
 // The 8th-order shapes without images and with PF 2 (in FP64 that of 16 columns) are held to 128 VGPRs (4 waves per
 // SIMD; FP32, 158k blocks: 3,347 us against 3,616 with 154 VGPRs and 3 waves); with image phases the shuffles push
-// every 8th-order shape past 168, so those are held to 168 (3 waves, 5 spills; at 128 they spill 53).  Measured, FP64,
+// every 8th-order shape past 168, so those are held to 168 (3 waves, 3 to 6 spills; at 128 they spill 53).  Measured, FP64,
 // 16 columns, 2 directions: 512 blocks at a k-point 49 -> 32 us, 1,024 blocks 87 -> 57, 6,144 blocks 705 -> 368 against
 // loading the other plane's lines as well; 45,896 blocks without images 2,118 -> 2,050 us from loading the potential
 // before the barrier.  16th order: unbounded (184 VGPRs; held to 168, 11,474 blocks FP64 take 941 us instead of 829).
@@ -1758,7 +1755,6 @@ int device_upload_plan(Plan const& p, DevicePlan& d, std::string& err) {
     }
     int s = 0;
     if ((s = dupload(d, d.colindx, p.colindx, err))) return s;
-    if ((s = dupload(d, d.rowindx, p.rowindx, err))) return s;
     if ((s = dupload(d, d.veff, p.veff_index, err))) return s;
     if ((s = dupload(d, d.row_pos, p.row_pos, err))) return s;
     {   // processing order of the local kernel: per source column, xy tiles of TILE x TILE target blocks swept
@@ -2231,8 +2227,7 @@ int device_action(DevicePlan& d, ActionScalars const& s, real_t* y, real_t const
             if (!n) continue;
             uint32_t const* bucket = d.bucket_chunks + d.bucket_start[L];
 #define LAUNCH_PRJ(LL) hipLaunchKernelGGL((k_sho_project<real_t, LL>), dim3(n), dim3(128), 0, stream, ws.partial, x, \
-                d.chunks, bucket, d.chunk_coef, d.prj_blocks, d.rowindx, d.row_pos, d.image_pos, \
-                s.hgrid[0], s.hgrid[1], s.hgrid[2], s.hgrid[3], d.col_active, d.htab, d.smask, d.prj_slot)
+                d.chunks, bucket, d.chunk_coef, d.prj_blocks, d.col_active, d.htab, d.smask, d.prj_slot)
 #define LAUNCH_MFMA(LL) hipLaunchKernelGGL((k_sho_project_mfma<real_t, LL>), dim3(n), dim3(256), 0, stream, ws.partial, \
                 x, d.chunks, bucket, d.chunk_coef, d.prj_blocks, d.col_active, d.htab, d.smask, d.prj_slot)
             if (d.prj_engine[sizeof(real_t) == 8 ? 0 : 1] == 1 && L <= 5) {   // the dense form on the matrix cores
@@ -2296,7 +2291,6 @@ int device_action(DevicePlan& d, ActionScalars const& s, real_t* y, real_t const
         for (int u = 0; u < 2; ++u) for (int v = 0; v < 2; ++v) a.phase[dd][u][v] = s.phase[dd][u][v];
     }
     a.cdiag = real_t(cdiag);
-    for (int k = 0; k < 4; ++k) a.hgrid[k] = s.hgrid[k];
     // work-groups are dealt round-robin to the 8 XCDs: give each XCD a contiguous range of
     // (block, column slice) items so that neighbour blocks meet in the same L2
     int const v = sizeof(real_t) == 8 ? 0 : 1;
@@ -2493,8 +2487,7 @@ template int device_autotune<float>(DevicePlan&, ActionScalars const&, float*, f
 // (h dVol-scaled, s dVol-scaled) before the SHO prefactors, see gfa_gradient).
 // projection of one FP64 vector onto every atom image and collection per (atom, column group) with the Bloch
 // phases: out[((atom_starts[a] + s) * nCols + c)][re/im][j]
-static int project_collect(DevicePlan& d, ActionScalars const& s, double const* vec, double* out, hipStream_t stream,
-                           std::string& err) {
+static int project_collect(DevicePlan& d, double const* vec, double* out, hipStream_t stream, std::string& err) {
     auto& ws = d.ws64;
     if (!ws.partial) {
         if (int r = dalloc(d, ws.partial, size_t(d.total_chunk_coefs) * 128, err)) return r;
@@ -2505,8 +2498,7 @@ static int project_collect(DevicePlan& d, ActionScalars const& s, double const* 
         if (!n) continue;
         uint32_t const* bucket = d.bucket_chunks + d.bucket_start[L];
 #define LAUNCH_PRJ(LL) hipLaunchKernelGGL((k_sho_project<double, LL>), dim3(n), dim3(128), 0, stream, ws.partial, vec, \
-        d.chunks, bucket, d.chunk_coef, d.prj_blocks, d.rowindx, d.row_pos, d.image_pos, \
-        s.hgrid[0], s.hgrid[1], s.hgrid[2], s.hgrid[3], (uint8_t const*)nullptr, d.htab, d.smask, d.prj_slot)
+        d.chunks, bucket, d.chunk_coef, d.prj_blocks, (uint8_t const*)nullptr, d.htab, d.smask, d.prj_slot)
         switch (L) {
             case 0: LAUNCH_PRJ(0); break; case 1: LAUNCH_PRJ(1); break;
             case 2: LAUNCH_PRJ(2); break; case 3: LAUNCH_PRJ(3); break;
@@ -2547,7 +2539,7 @@ int device_density_matrices(DevicePlan& d, Plan const& p, ActionScalars const& s
         std::fill(D, D + w.n, 0.0);
         return 0;
     }
-    if (int r = project_collect(d, s, X, d.atom_coef, stream, err)) return r;
+    if (int r = project_collect(d, X, d.atom_coef, stream, err)) return r;
     hipLaunchKernelGGL(k_density, dim3(d.nAtomImages, d.max_atom_nc), dim3(256), 0, stream, w.D, d.atom_coef, d.image_pos,
                        d.image_lmax, d.image_phase, w.desc, d.nAtomImages, d.nCols, s.hgrid[0], s.hgrid[1], s.hgrid[2],
                        s.hgrid[3], factor);
@@ -2589,7 +2581,7 @@ int device_gradient(DevicePlan& d, Plan const& p, ActionScalars const& s, double
     HIP_TRY(hipGetLastError());
     if (d.nAtoms > 0 && d.nchunks > 0) {
         for (int v = 0; v < 2; ++v)
-            if (int r = project_collect(d, s, v ? Lam : X, v ? g.cL : g.cX, stream, err)) return r;
+            if (int r = project_collect(d, v ? Lam : X, v ? g.cL : g.cX, stream, err)) return r;
         hipLaunchKernelGGL(k_grad_atoms, dim3(d.nAtoms, d.max_atom_nc, (d.max_atom_nc + 3) / 4), dim3(256), 0, stream, g.gmat, g.cX, g.cL,
                            d.atom_lmax, d.atom_starts, d.atom_mat_off, g.wE, d.nCols);
         HIP_TRY(hipGetLastError());

@@ -66,7 +66,6 @@ struct DevicePlan {
 
     // index data
     uint16_t* colindx = nullptr;       // [nnzb]
-    uint32_t* rowindx = nullptr;       // [nnzb]
     int32_t* veff = nullptr;           // [nnzb]
     // per-block headers of the local kernels, head_words (16, or 32 when nh_max = 2) words each: the block, its
     // column group, potential cell, add-list range and neighbour codes [direction][side][k], so that a work-group
